@@ -22,10 +22,11 @@
 // Kernels
 //   bwd_rows_vec -- channel-first rows, same lane layout and item order as
 //                   fwd_rows_vec (one item per wavefront, 4 per block),
-//                   ragged rows included: positions count from the 16-byte
-//                   boundary at or before the row's first element (the row is
-//                   [m, m + L)), dpre is zero outside the row, and the vectors
-//                   shared with neighbouring rows are stored element by element.
+//                   rows of any start and length included (RowsMode in
+//                   cc1d_device.hpp): dpre is zero outside the row, and a row's
+//                   first and last few elements are stored in smaller pieces.
+//   bwd_rows_short - rows of at most 32 vectors: a wavefront takes as many
+//                   whole rows as fit into its 64 lanes, a lane one vector.
 //   bwd_clw      -- channel-last (unit channel stride); a lane owns 4 bytes of
 //                   adjacent channels, a wavefront walks a run of time steps.
 //   bwd_generic  -- any strides; one thread per (b, c, chunk of time).
@@ -37,14 +38,14 @@ namespace cc1d {
 
 struct BwdArgs {
     cc1d_bwd_params p;
-    FastDiv nseg_div;  // rows_vec: item -> row
+    FastDiv nseg_div;  // rows_vec: item -> row; rows_short: lane -> row of the wavefront
     FastDiv dim_div;   // rows_vec: row -> batch entry
     float* part;      // non-null: write weight/bias-gradient partial sums here instead of atomics
     int64_t nseg;     // rows_vec: segments per row; cl: run groups per row; generic: chunks per row
-    int64_t n_items;  // rows_vec: (row, segment) items; generic: threads
-    int64_t chunk;    // cl: time steps per run; generic: time steps per thread
+    int64_t n_items;  // rows_vec: (row, segment) items; rows_short: rows; generic: threads
+    int64_t chunk;    // cl: time steps per run; generic: time steps per thread; rows_short: rows per wavefront
     int64_t groups;   // cl: channel groups of 64 * CPL
-    int32_t ragged;   // rows_vec: rows may start off a 16-byte boundary / end inside a vector (kernel variant)
+    int32_t nvec;     // rows_short: vectors per row
 };
 
 // channel-first rows: (row, segment) items per block, one per wavefront
@@ -55,54 +56,150 @@ constexpr int kClR = 128;      // run length, and the shorter ones for small gri
 constexpr int kClRMid = 64;
 constexpr int kClRShort = 16;
 constexpr int kClWPB = 8;
+// generic: time steps per thread
+constexpr int kGenericChunk = 64;
 
 // Registers of one wavefront-segment of a row: VPT 16-byte vectors of x and
-// dout per lane, plus the wave-uniform halos (scalar registers): the vector
-// of x before the segment (used by lane 0) and x and dout of the first vector
-// after it (used by lane 63); zero past either end of the row.
+// dout per lane, plus the halos: the vector of x before the segment (used by
+// lane 0) and x and dout of the first vector after it (used by lane 63); zero
+// past either end of the row. Wave-uniform (scalar registers) where vectors
+// are aligned; in kRowsAny h and xn are one register vector per lane, lane 0's
+// being h (as single elements in scalar registers they cost more: 106 instead
+// of 104 vector registers at bf16, W 4, and scratch memory at W 9).
 template <int VPT> struct RowTile {
     u32x4 v[VPT], gv[VPT], h, xn, gn;
 };
 
+// A value that is read through the scalar cache where its address is the same
+// for the whole wavefront.
+template <bool UNIFORM, typename T> __device__ __forceinline__ float ld_row(const T* p) {
+    if constexpr (UNIFORM) return ld_uniform(p);
+    else return to_f32(*p);
+}
+
+// Positions of a row count from m elements before its first: it is
+// [m, m + L), m 0 except in kRowsAlike.
+//
 // Issue the loads of segment t0 of row (b, c). FULL: the whole segment lies
-// inside the row.
-template <typename T, int VPT, bool FULL>
+// inside the row. L: the row's end (0 for a lane without a row). kRowsAlike
+// reads whole aligned vectors, a neighbouring row's elements in the row's
+// first and last one included.
+template <typename T, int VPT, bool FULL, int MODE>
 __device__ __forceinline__ void bwd_rows_load(const cc1d_bwd_params& p, int lane, int64_t b, int64_t c, int32_t t0,
-                                              int32_t m, RowTile<VPT>& r) {
+                                              int32_t L, int32_t m, RowTile<VPT>& r) {
     constexpr int EPV = elems16<T>::value;
     constexpr int SEG = 64 * VPT * EPV;
-    const int32_t L = (int32_t)p.seqlen + m;  // the row's end (its start is m)
     const int32_t tn = t0 + SEG;  // first position of the next segment
     const T* __restrict__ xr = static_cast<const T*>(p.x) + b * p.x_stride[0] + c * p.x_stride[1] - m;
     const T* __restrict__ gr = static_cast<const T*>(p.dout) + b * p.dout_stride[0] + c * p.dout_stride[1] - m;
+    if constexpr (MODE == kRowsAligned || MODE == kRowsAlike) {
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-        const int32_t t = t0 + (j * 64 + lane) * EPV;
-        r.v[j] = (FULL || t < L) ? vload_nt(xr + t) : vzero();
-        r.gv[j] = (FULL || t < L) ? vload_nt(gr + t) : vzero();
+        for (int j = 0; j < VPT; ++j) {
+            const int32_t t = t0 + (j * 64 + lane) * EPV;
+            r.v[j] = (FULL || t < L) ? vload_nt(xr + t) : vzero();
+            r.gv[j] = (FULL || t < L) ? vload_nt(gr + t) : vzero();
+        }
+        // halo vectors: wave-uniform reads at clamped (always valid) addresses
+        const u32x4 hv = vload_uniform(xr + (t0 > 0 ? t0 - EPV : 0));
+        const int32_t tq = tn < L ? tn : t0;
+        const u32x4 xv = vload_uniform(xr + tq), gq = vload_uniform(gr + tq);
+        r.h = t0 > 0 ? hv : vzero();
+        r.xn = tn < L ? xv : vzero();
+        r.gn = tn < L ? gq : vzero();
+    } else {
+        // the halos first: lane 0 needs its one for the first vector's arithmetic
+        u32x4 e = vzero(), ge = vzero();
+        const int rem = (int32_t)p.seqlen & (EPV - 1);
+        if constexpr (MODE == kRowsAny) {
+            if (lane == 0 && t0 > 0) e = vload_any(xr + (t0 - EPV));
+            if (tn + EPV <= L) {  // wave-uniform
+                if (lane == 63) {
+                    e = vload_any(xr + tn);
+                    ge = vload_any(gr + tn);
+                }
+            } else if (tn < L) {  // the next segment is the row's last few elements
+                if (lane == 63) {
+                    RowTail<T> xt, gt;
+                    xt.load(xr + tn, rem);
+                    gt.load(gr + tn, rem);
+                    e = xt.vec(rem);
+                    ge = gt.vec(rem);
+                }
+            }
+        }
+        r.h = r.xn = e;
+        r.gn = ge;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int32_t t = t0 + (j * 64 + lane) * EPV;
+            r.v[j] = (FULL || t + EPV <= L) ? vload_any_nt(xr + t) : vzero();
+            r.gv[j] = (FULL || t + EPV <= L) ? vload_any_nt(gr + t) : vzero();
+        }
+        if (!FULL && rem != 0) {  // wave-uniform: the row's last rem elements
+            const int32_t tp = (int32_t)p.seqlen - rem;
+            const int jt = MODE == kRowsShort ? 0 : (tp - t0) / (64 * EPV);
+            if (tp >= t0) {  // wave-uniform
+                RowTail<T> xt, gt;
+                xt.a = gt.a = u32x2{0u, 0u};
+                xt.b = xt.c = gt.b = gt.c = 0u;
+                if (tp == t0 + (jt * 64 + lane) * EPV && tp < L) {
+                    xt.load(xr + tp, rem);
+                    gt.load(gr + tp, rem);
+                }
+                const u32x4 xv = xt.vec(rem), gq = gt.vec(rem);  // zero in the other lanes
+#pragma unroll
+                for (int j = 0; j < VPT; ++j)
+                    if (j == jt) {
+                        r.v[j] |= xv;
+                        r.gv[j] |= gq;
+                    }
+            }
+        }
     }
-    // halo vectors: wave-uniform reads at clamped (always valid) addresses
-    const u32x4 hv = vload_uniform(xr + (t0 > 0 ? t0 - EPV : 0));
-    const int32_t tq = tn < L ? tn : t0;
-    const u32x4 xv = vload_uniform(xr + tq), gq = vload_uniform(gr + tq);
-    r.h = t0 > 0 ? hv : vzero();
-    r.xn = tn < L ? xv : vzero();
-    r.gn = tn < L ? gq : vzero();
 }
+
+// Store vector o of dx at position t (dxr: the row), the part of it that
+// lies inside the row.
+template <typename T, bool FULL, int MODE>
+__device__ __forceinline__ void bwd_rows_store(T* dxr, int32_t t, int32_t m, int32_t L, const float* o) {
+    constexpr int EPV = elems16<T>::value;
+    const u32x4 ov = vpack<T>(o);
+    if constexpr (MODE == kRowsAligned) {
+        if (FULL || t < L) vstore_nt(dxr + t, ov);
+    } else if constexpr (MODE == kRowsAlike) {
+        if (FULL || (t >= m && t + EPV <= L)) {
+            vstore_nt(dxr + t, ov);
+        } else if (t < L) {  // a vector shared with a neighbouring row
+#pragma unroll
+            for (int e = 0; e < EPV; ++e)
+                if ((uint32_t)(t + e - m) < (uint32_t)(L - m)) st_elem<T>(dxr + t + e, ov, e);
+        }
+    } else {
+        if (FULL || t + EPV <= L) vstore_any_nt(dxr + t, ov);
+        else if (t < L) RowTail<T>::store(dxr + t, ov, L - t);
+    }
+}
+
+// Id of a position outside its row: a lane's sequence id there differs from
+// every id a row has (of any sign), so that no tap of it is kept.
+constexpr int32_t kNoId = INT32_MIN;
 
 // One wavefront-segment of row (b, c) from its loaded tile, without seq_idx
 // (bwd_rows_compute_seq below has it): writes dx (and dinitial_states) and
-// adds this segment's weight/bias-gradient partials into pw / pb. RAG: the
-// row starts m elements past a 16-byte boundary (m is 0 otherwise).
-template <typename T, int W, int VPT, bool SILU, bool FULL, bool RAG>
-__device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int lane, int64_t b, int64_t c,
-                                                 int32_t t0, int32_t m, RowTile<VPT> r, const float* w,
-                                                 const float* wq, float bq, float* pw, float& pb) {
+// adds this segment's weight/bias-gradient partials into pw / pb. L: the
+// row's end (kRowsShort: 0 in a lane without a row); lastl: the row's last
+// lane (63 unless kRowsShort).
+template <typename T, int W, int VPT, bool SILU, bool FULL, int MODE>
+__device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int lane, int lastl, int64_t b, int64_t c,
+                                                 int32_t t0, int32_t L, int32_t m, RowTile<VPT> r,
+                                                 const float* w, const float* wq, float bq, float* pw, float& pb) {
     constexpr int EPV = elems16<T>::value;
     constexpr int H = W - 1;
     constexpr int SEG = 64 * VPT * EPV;
+    constexpr bool SHORT = MODE == kRowsShort, ALIKE = MODE == kRowsAlike;
+    constexpr bool EDGES = MODE != kRowsAligned && !FULL;  // the row may start or end inside a vector
     static_assert(H <= EPV, "the halo must fit in one 16-byte vector");
-    const int32_t L = (int32_t)p.seqlen + m;  // the row is [m, L) in this segment's positions
+    const int32_t Lr = (int32_t)p.seqlen + m;  // L in every lane that has a row
     {
         const int32_t tn = t0 + SEG;  // first position of the next segment
         T* __restrict__ dxr = static_cast<T*>(p.dx) + b * p.dx_stride[0] + c * p.dx_stride[1] - m;
@@ -116,25 +213,25 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
             const T* is = static_cast<const T*>(p.initial_states) + b * p.initial_states_stride[0] +
                           c * p.initial_states_stride[1];
 #pragma unroll
-            for (int i = 0; i < H; ++i) hinit[i] = ld_uniform(is + i * p.initial_states_stride[2]);
+            for (int i = 0; i < H; ++i) hinit[i] = ld_row<!SHORT>(is + i * p.initial_states_stride[2]);
         }
         // dfinal_states of this row when the segment holds one of the row's
-        // last W-1 positions (wave-uniform; a ragged row's may span two
-        // segments, an aligned row's lie in its last vector)
+        // last W-1 positions (wave-uniform; they may span two segments, an
+        // aligned row's lie in its last vector)
         float dfin[H];
 #pragma unroll
         for (int i = 0; i < H; ++i) dfin[i] = 0.0f;
-        const bool dfin_row = p.dfinal_states != nullptr && tn > L - H;
+        const bool dfin_row = p.dfinal_states != nullptr && tn > Lr - H;
         if (dfin_row) {
             const T* dfs = static_cast<const T*>(p.dfinal_states) + b * p.dfinal_states_stride[0] +
                            c * p.dfinal_states_stride[1];
 #pragma unroll
-            for (int i = 0; i < H; ++i) dfin[i] = ld_uniform(dfs + i * p.dfinal_states_stride[2]);
+            for (int i = 0; i < H; ++i) dfin[i] = ld_row<!SHORT>(dfs + i * p.dfinal_states_stride[2]);
         }
-        // a ragged row's first vector holds m elements of the previous row:
-        // they are positions -m .. -1 of this one (x: initial_states or zero;
-        // dout: zero), merged in as raw bits
-        if (RAG && !FULL && t0 == 0 && m > 0 && lane == 0) {
+        // the first vector's m elements of the previous row are positions
+        // -m .. -1 of this one (x: initial_states or zero; dout: zero), merged
+        // in as raw bits
+        if (ALIKE && !FULL && t0 == 0 && m > 0 && lane == 0) {
             constexpr int EPD = EPV / 4;  // elements per dword
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
@@ -149,15 +246,14 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
         }
         const auto& v = r.v;
         const auto& gv = r.gv;
-        const u32x4 h = r.h, xn = r.xn, gn = r.gn;
-
         // The vectors are processed in order: dpre of vector j (with its
         // gradient partials), then dx of vector j - 1, which needs dpre of
         // vector j only for lane 63's last H positions (lane 0's first H). So
         // two vectors of dpre are live at a time, not the whole segment.
         constexpr int D0 = ((EPV - H) * (int)sizeof(T)) / 4;
-        const int prev_lane = (lane + 63) & 63;
-        const int next_lane = (lane + 1) & 63;
+        const int wl = SHORT ? (int)(threadIdx.x & 63) : lane;  // lane of the wavefront
+        const int prev_lane = (wl + 63) & 63;
+        const int next_lane = (wl + 1) & 63;
 
         // ---- dpre of vector j + dweight/dbias partials ----
         // PART: some lane's vector j may hold a position outside the row
@@ -167,21 +263,21 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
             u32x4 pv = vzero();
 #pragma unroll
             for (int d = D0; d < 4; ++d) {
-                const uint32_t send = (lane == 63) ? (j > 0 ? v[j > 0 ? j - 1 : 0][d] : 0u) : v[j][d];
+                const uint32_t send = (!SHORT && lane == 63) ? (j > 0 ? v[j > 0 ? j - 1 : 0][d] : 0u) : v[j][d];
                 pv[d] = lane_get(send, prev_lane);
             }
-            if (j == 0 && lane == 0) pv = h;
+            if (j == 0 && lane == 0) pv = SHORT ? vzero() : r.h;
             // an aligned row's first vector past its end: its window reads
             // zero too, so that no x of the row meets that vector's zero dpre
             // (zero times a non-finite x would be NaN)
-            if (!FULL && !RAG && t >= L) pv = vzero();
+            if (!FULL && MODE == kRowsAligned && t >= L) pv = vzero();
             float win[H + EPV];
 #pragma unroll
             for (int i = 0; i < H; ++i) {
-                if constexpr (FULL || !RAG)  // m == 0 whenever a first segment is full
-                    win[i] = (j == 0 && use_init) ? hinit[i] : vget<T>(pv, EPV - H + i);
-                else  // before the row: position i - H - m, initial_states slot i - m
+                if constexpr (ALIKE && !FULL)  // before the row: position i - H, initial_states slot i - m
                     win[i] = (j == 0 && use_init) ? pick<H>(hinit, i - m) : vget<T>(pv, EPV - H + i);
+                else  // m == 0 whenever a first segment is full
+                    win[i] = (j == 0 && use_init) ? hinit[i] : vget<T>(pv, EPV - H + i);
             }
 #pragma unroll
             for (int i = 0; i < EPV; ++i) win[H + i] = vget<T>(v[j], i);
@@ -200,14 +296,14 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
                 // to the weight gradient (a select, not a product with zero,
                 // which a non-finite x there would turn into NaN). Aligned
                 // rows end on a vector boundary: the test is the vector's.
-                const bool outside = PART && (RAG ? (t + i < m || t + i >= L) : t >= L);
+                const bool outside = PART && (EDGES ? (t + i < m || t + i >= L) : t >= L);
                 if (outside) d = 0.0f;
                 dpj[i] = d;
                 pb += d;
 #pragma unroll
                 for (int k = 0; k < W; ++k) {
                     const float s = __builtin_fmaf(d, win[i + k], pw[k]);
-                    pw[k] = (RAG && outside) ? pw[k] : s;
+                    pw[k] = (EDGES && outside) ? pw[k] : s;
                 }
             }
         };
@@ -222,9 +318,9 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
             for (int i = 0; i < EPV; ++i) de[i] = dpj[i];
 #pragma unroll
             for (int i = 0; i < H; ++i) {
-                const float send = (lane == 0) ? (lastv ? 0.0f : dpn[i]) : dpj[i];
+                const float send = (!SHORT && lane == 0) ? (lastv ? 0.0f : dpn[i]) : dpj[i];
                 const float r = lane_get(send, next_lane);
-                de[EPV + i] = (lane == 63 && lastv) ? dpn[i] : r;
+                de[EPV + i] = (lane == lastl && lastv) ? dpn[i] : r;
             }
             float o[EPV];
 #pragma unroll
@@ -239,48 +335,37 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
             // branch skips it for every segment without the row end (as a
             // lane-masked block it was issued, empty, by all of them).
             if (dfin_row) {
-                if constexpr (!RAG) {  // the row's last vector ends with them
+                if constexpr (MODE == kRowsAligned) {  // the row's last vector ends with them
                     const bool last = t + EPV == L;
 #pragma unroll
                     for (int i = EPV - H; i < EPV; ++i) {
                         const float v = round_to<T>(o[i]) + dfin[H - EPV + i];
                         o[i] = last ? v : o[i];
                     }
-                } else {
+                } else if (t0 + (j + 1) * 64 * EPV > Lr - H) {  // wave-uniform: some lane's vector j holds one
 #pragma unroll
                     for (int i = 0; i < EPV; ++i) {
                         const int32_t pos = t + i;
                         const float v = round_to<T>(o[i]) + pick<H>(dfin, pos - L + H);
-                        o[i] = (pos >= L - H && pos < L && pos >= m) ? v : o[i];
+                        o[i] = (pos >= L - H && pos < L) ? v : o[i];
                     }
                 }
             }
-            if constexpr (!RAG) {
-                if (FULL || t < L) vstore_nt(dxr + t, vpack<T>(o));
-            } else {
-                const u32x4 ov = vpack<T>(o);
-                if (FULL || (t >= m && t + EPV <= L)) {
-                    vstore_nt(dxr + t, ov);
-                } else if (t < L) {  // a vector shared with a neighbouring row
-#pragma unroll
-                    for (int e = 0; e < EPV; ++e)
-                        if ((uint32_t)(t + e - m) < (uint32_t)p.seqlen) st_elem<T>(dxr + t + e, ov, e);
-                }
-            }
+            bwd_rows_store<T, FULL, MODE>(dxr, t, m, L, o);
         };
 
         float dp[2][EPV];
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            if constexpr (RAG && !FULL && SILU) {
+            if constexpr (EDGES && SILU) {
                 // With SiLU, x and dout zeroed past the row's end (and before its
                 // start, above) make every outside position's dpre an exact zero
                 // whenever the row's own values are finite; where they are not,
                 // the reference's weight and bias gradients are NaN as well (the
                 // SiLU derivative at a non-finite pre is NaN). So no position
-                // needs a mask of its own. Wave-uniform test: vector j may hold
-                // positions past the end.
-                if (t0 + (j + 1) * 64 * EPV > L) {
+                // needs a mask of its own. (What a lane without a row computes
+                // from its neighbour's window is dropped.)
+                if (ALIKE && t0 + (j + 1) * 64 * EPV > L) {  // wave-uniform: vector j may reach past the end
                     const int32_t t = t0 + (j * 64 + lane) * EPV;
 #pragma unroll
                     for (int d = 0; d < 4; ++d) {
@@ -290,23 +375,22 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
                     }
                 }
                 dpre_vec(j, dp[j & 1], std::false_type{});
-            } else if constexpr (RAG && !FULL) {
-                // a ragged row's segments are not full, but only their first and
-                // last vectors hold positions outside the row (wave-uniform test)
+            } else if constexpr (EDGES) {
+                // only the vectors that hold the row's ends need the masks (wave-uniform test)
                 const int32_t vs = t0 + j * 64 * EPV;  // vector j of lane 0
-                if (vs >= m && vs + 64 * EPV <= L) dpre_vec(j, dp[j & 1], std::false_type{});
+                if (vs >= m && vs + 64 * EPV <= Lr) dpre_vec(j, dp[j & 1], std::false_type{});
                 else dpre_vec(j, dp[j & 1], std::true_type{});
             } else {
                 dpre_vec(j, dp[j & 1], std::bool_constant<!FULL>{});
             }
             if (j == 0 && p.dinitial_states != nullptr && t0 == 0) {  // wave-uniform
-                // dinitial_states (bwd_full_cpu/kernel.mojo:210-219) from dpre of
-                // positions 0 .. H-1: elements m .. m+H-1 of lane 0's first
+                // dinitial_states (bwd_full_cpu/kernel.mojo:210-219) from dpre of the
+                // row's first H positions: elements m .. m+H-1 of lane 0's first
                 // vector, the ones past its end in lane 1's
                 float d0[H];
 #pragma unroll
                 for (int q = 0; q < H; ++q) {
-                    if constexpr (FULL || !RAG) {
+                    if constexpr (FULL || !ALIKE) {
                         d0[q] = dp[0][q];
                     } else {
                         const float own = pick<EPV>(dp[0], m + q);
@@ -315,7 +399,7 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
                         d0[q] = m + q < EPV ? own : nxt;
                     }
                 }
-                if (lane == 0) {
+                if (lane == 0 && L > 0) {
                     T* di = static_cast<T*>(p.dinitial_states) + b * p.dinitial_states_stride[0] +
                             c * p.dinitial_states_stride[1];
 #pragma unroll
@@ -335,16 +419,16 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
         float dn[H];
 #pragma unroll
         for (int i = 0; i < H; ++i) dn[i] = 0.0f;
-        if (tn < L) {
+        if (!SHORT && tn < L) {
             float xw[2 * H];
 #pragma unroll
             for (int i = 0; i < H; ++i) {
                 xw[i] = vget<T>(v[VPT - 1], EPV - H + i);
-                xw[H + i] = vget<T>(xn, i);
+                xw[H + i] = vget<T>(r.xn, i);
             }
 #pragma unroll
             for (int i = 0; i < H; ++i) {
-                const float g = vget<T>(gn, i);
+                const float g = vget<T>(r.gn, i);
                 float d = g;
                 if constexpr (SILU) {
                     float q = bq;
@@ -372,72 +456,79 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
 // carry that the owning lane fetches from its neighbour (lane 63: from lane
 // 0 of the next vector, or from the next segment's first H positions); each
 // dx sum is the gather's fma chain with that carry added as one term.
-template <typename T, int W, int VPT, bool SILU, bool FULL, bool RAG>
-__device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, int lane, int64_t b, int64_t c,
-                                                     int32_t t0, int32_t m, RowTile<VPT> r,
+template <typename T, int W, int VPT, bool SILU, bool FULL, int MODE>
+__device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, int lane, int lastl, int64_t b,
+                                                     int64_t c, int32_t t0, int32_t L, int32_t m, RowTile<VPT> r,
                                                      const float* w, const float* wq, float bq, float* pw,
                                                      float& pb) {
     constexpr int EPV = elems16<T>::value;
     constexpr int H = W - 1;
     constexpr int SEG = 64 * VPT * EPV;
+    constexpr bool SHORT = MODE == kRowsShort, ALIKE = MODE == kRowsAlike;
+    constexpr bool EDGES = MODE != kRowsAligned && !FULL;  // the row may start or end inside a vector
     static_assert(H <= EPV, "the halo must fit in one 16-byte vector");
     constexpr int D0 = ((EPV - H) * (int)sizeof(T)) / 4;
-    const int32_t Lr = (int32_t)p.seqlen;  // the row's length
-    const int32_t L = Lr + m;              // its end: the row is [m, L) in these positions
-    const int32_t tn = t0 + SEG;  // first position of the next segment
+    const int32_t Lr = (int32_t)p.seqlen + m;  // L in every lane that has a row
+    const int32_t tn = t0 + SEG;               // first position of the next segment
+    const int rem = Lr & (EPV - 1);
     T* __restrict__ dxr = static_cast<T*>(p.dx) + b * p.dx_stride[0] + c * p.dx_stride[1] - m;
-    const int32_t* __restrict__ sr = p.seq_idx + b * p.seq_idx_stride[0];
-    // (unit time stride) ragged rows: a vector's ids start rid ids past a
-    // 16-byte boundary (its first position, t - m, is a multiple of 4 plus
-    // -m); the row's first id a0 past one
-    const int a0 = RAG ? (int)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(sr) / 4) & 3u) : 0;
-    const int rid = (a0 - m) & 3;
-    const int prev_lane = (lane + 63) & 63;
-    const int next_lane = (lane + 1) & 63;
-    // a ragged row's first vector holds m elements of the previous row: x
-    // there reads as zero, as before an aligned row (a padding position's id
-    // matches theirs, -1, and a tap is kept by its id alone)
-    if (RAG && !FULL && t0 == 0 && m > 0 && lane == 0) {
-        float fx[EPV];
+    const int32_t* __restrict__ sr = p.seq_idx + b * p.seq_idx_stride[0] - m;  // unit time stride
+    const int wl = SHORT ? (int)(threadIdx.x & 63) : lane;                     // lane of the wavefront
+    const int prev_lane = (wl + 63) & 63;
+    const int next_lane = (wl + 1) & 63;
+    // the first vector's m elements of the previous row: x there reads as
+    // zero, as before an aligned row (a padding position's id matches theirs,
+    // -1, and a tap is kept by its id alone)
+    if (ALIKE && !FULL && t0 == 0 && m > 0 && lane == 0) {
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) fx[e] = e >= m ? vget<T>(r.v[0], e) : 0.0f;
-        r.v[0] = vpack<T>(fx);
+        for (int d = 0; d < 4; ++d) r.v[0][d] &= ~lead_mask<T>(d, m);
     }
 
-    // ids: the lane's positions (-1 outside the row), and the H before and
+    // x past the row's end reads as zero (the other modes have it so)
+    if constexpr (ALIKE && !FULL) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+            if (t0 + (j + 1) * 64 * EPV > L) {  // wave-uniform: vector j may reach past the end
+                const int32_t t = t0 + (j * 64 + lane) * EPV;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) r.v[j][d] &= lead_mask<T>(d, L - t);
+            }
+    }
+
+    // ids: the lane's positions (kNoId outside the row), and the H before and
     // after the segment (wave-uniform, -1 outside the row)
     int32_t id[VPT][EPV];
-    IdsRaw<EPV> raw[RAG ? VPT : 1];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int32_t t = t0 + (j * 64 + lane) * EPV;
-        if constexpr (!RAG) {  // 16-byte vectors of 4 ids
+        if constexpr (MODE == kRowsAligned) {  // 16-byte vectors of 4 ids
 #pragma unroll
             for (int q = 0; q < EPV / 4; ++q) {
-                const u32x4 sv = (FULL || t < L) ? *reinterpret_cast<const u32x4*>(sr + t + 4 * q)
-                                                 : u32x4{0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+                constexpr uint32_t no = (uint32_t)kNoId;
+                const u32x4 sv = (FULL || t < L) ? *reinterpret_cast<const u32x4*>(sr + t + 4 * q) : u32x4{no, no, no, no};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) id[j][4 * q + e] = (int32_t)sv[e];
             }
         } else {
-            ids_load<EPV, !FULL>(sr, Lr, t - m, rid, a0, raw[j]);
-        }
-    }
-    if constexpr (RAG) {  // -1 outside the row
 #pragma unroll
-        for (int j = 0; j < VPT; ++j) {
-            const int32_t pos = t0 + (j * 64 + lane) * EPV - m;
-            const int32_t vs = t0 + j * 64 * EPV;  // vector j of lane 0: inside the row in every lane?
-            if (FULL || (vs >= m && vs + 64 * EPV <= L)) ids_shift<EPV, false>(raw[j], Lr, pos, rid, id[j]);
-            else ids_shift<EPV, true>(raw[j], Lr, pos, rid, id[j]);
+            for (int e = 0; e < EPV; ++e) id[j][e] = kNoId;
+            if (FULL || (t >= m && t + EPV <= L)) ids_any<EPV>(sr + t, id[j]);
+            // a row's first and last few ids, each into its own register (no
+            // wait here); wave-uniform tests around
+            if (ALIKE && !FULL && j == 0 && t0 == 0 && m > 0) {
+                if (lane == 0) ids_some<EPV>(sr, m, EPV, id[0]);
+            }
+            if (EDGES && rem != 0 && (SHORT || t0 + (j + 1) * 64 * EPV > Lr)) {
+                if (t < L && t + EPV > L) ids_some<EPV>(sr + t, 0, rem, id[j]);
+            }
         }
     }
     int32_t hid[H], nid[H];
 #pragma unroll
     for (int i = 0; i < H; ++i) {
-        const int32_t ph = t0 - H + i - m, pn = tn + i - m;  // row positions
-        hid[i] = ph >= 0 ? ld_uniform(sr + ph) : -1;
-        nid[i] = pn < Lr ? ld_uniform(sr + pn) : -1;
+        const int32_t ph = t0 - H + i, pn = tn + i;
+        hid[i] = !SHORT && ph >= m ? ld_uniform(sr + ph) : -1;
+        nid[i] = !SHORT && pn < Lr ? ld_uniform(sr + pn) : -1;
     }
 
     float acc[2][EPV];  // dx sums of the lane's positions, by vector parity
@@ -450,20 +541,12 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
         const int32_t t = t0 + (j * 64 + lane) * EPV;
 #pragma unroll
         for (int i = 0; i < H; ++i) {
-            const float send = (lane == 0 && !local) ? nxt[i] : cj[i];
+            const float send = (!SHORT && lane == 0 && !local) ? nxt[i] : cj[i];
             float rv = lane_get(send, next_lane);
-            if (local && lane == 63) rv = nxt[i];
+            if (local && lane == lastl) rv = nxt[i];
             a[EPV - H + i] += rv;
         }
-        if constexpr (!RAG) {
-            if (FULL || t < L) vstore_nt(dxr + t, vpack<T>(a));
-        } else if (FULL || (t >= m && t + EPV <= L)) {
-            vstore_nt(dxr + t, vpack<T>(a));
-        } else if (t < L) {  // a vector shared with a neighbouring row
-#pragma unroll
-            for (int e = 0; e < EPV; ++e)
-                if (t + e >= m && t + e < L) st(dxr, t + e, a[e]);
-        }
+        bwd_rows_store<T, FULL, MODE>(dxr, t, m, L, a);
     };
 
 #pragma unroll
@@ -473,17 +556,17 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
         u32x4 pv = vzero();
 #pragma unroll
         for (int d = D0; d < 4; ++d) {
-            const uint32_t send = (lane == 63) ? (j > 0 ? r.v[j > 0 ? j - 1 : 0][d] : 0u) : r.v[j][d];
+            const uint32_t send = (!SHORT && lane == 63) ? (j > 0 ? r.v[j > 0 ? j - 1 : 0][d] : 0u) : r.v[j][d];
             pv[d] = lane_get(send, prev_lane);
         }
-        if (j == 0 && lane == 0) pv = r.h;
+        if (j == 0 && lane == 0) pv = SHORT ? vzero() : r.h;
         float win[H + EPV];
         int32_t iw[H + EPV];
 #pragma unroll
         for (int i = 0; i < H; ++i) {
             win[i] = vget<T>(pv, EPV - H + i);
-            const int32_t send = (lane == 63) ? (j > 0 ? id[j > 0 ? j - 1 : 0][EPV - H + i] : -1)
-                                              : id[j][EPV - H + i];
+            const int32_t send = (!SHORT && lane == 63) ? (j > 0 ? id[j > 0 ? j - 1 : 0][EPV - H + i] : -1)
+                                                        : id[j][EPV - H + i];
             const int32_t rv = lane_get(send, prev_lane);
             iw[i] = (j == 0 && lane == 0) ? hid[i] : rv;
         }
@@ -519,15 +602,13 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
                 for (int kk = 0; kk < W; ++kk) q = __builtin_fmaf(wq[kk], xe[kk], q);
                 d = silu_bwd_q(g, q);
             }
-            // outside the row: nothing added (a select, as in bwd_rows_compute)
-            const bool outside = !FULL && (RAG ? (t + e < m || t + e >= L) : t + e >= L);
-            if (outside || cur < 0) d = 0.0f;
+            // padding, and outside the row: there every x is zero too (no tap
+            // before is kept, its own x reads as zero), so that nothing is added
+            // whatever the row holds
+            if (cur < 0) d = 0.0f;
             pb += d;
 #pragma unroll
-            for (int kk = 0; kk < W; ++kk) {
-                const float s = __builtin_fmaf(d, xe[kk], pw[kk]);
-                pw[kk] = outside ? pw[kk] : s;
-            }
+            for (int kk = 0; kk < W; ++kk) pw[kk] = __builtin_fmaf(d, xe[kk], pw[kk]);
             // dx[s - k] += w[W-1-k] * dpre[s] where tap W-1-k of s is kept
 #pragma unroll
             for (int k = 0; k <= H; ++k) {
@@ -551,7 +632,7 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
     float cn[H];
 #pragma unroll
     for (int i = 0; i < H; ++i) cn[i] = 0.0f;
-    if (tn < L) {
+    if (!SHORT && tn < L) {
         float xw[2 * H];
         int32_t iw[2 * H];
 #pragma unroll
@@ -592,29 +673,36 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
 // always valid, so no branch holds them apart), which all complete before
 // the arithmetic starts -- the empty asm uses their values, so the compiler
 // can neither sink a load into the arithmetic nor wait for each on its own.
-template <typename T, int W, int VPT, bool SILU, bool SEQ, bool FULL, bool RAG>
-__device__ __forceinline__ void bwd_rows_item(const cc1d_bwd_params& p, int lane, int64_t b, int64_t c, int32_t t0,
-                                              int32_t m, float* pw, float& pb) {
+template <typename T, int W, int VPT, bool SILU, bool SEQ, bool FULL, int MODE>
+__device__ __forceinline__ void bwd_rows_item(const cc1d_bwd_params& p, int lane, int lastl, int64_t b, int64_t c,
+                                              int32_t t0, int32_t L, int32_t m, float* pw, float& pb) {
+    constexpr bool SHORT = MODE == kRowsShort;
     RowTile<VPT> r;
-    bwd_rows_load<T, VPT, FULL>(p, lane, b, c, t0, m, r);
+    bwd_rows_load<T, VPT, FULL, MODE>(p, lane, b, c, t0, L, m, r);
     float w[W];
     const T* __restrict__ wr = static_cast<const T*>(p.weight) + c * p.weight_stride[0];
 #pragma unroll
-    for (int k = 0; k < W; ++k) w[k] = ld_uniform(wr + k * p.weight_stride[1]);
+    for (int k = 0; k < W; ++k) w[k] = ld_row<!SHORT>(wr + k * p.weight_stride[1]);
     const T* br = p.bias ? static_cast<const T*>(p.bias) + c * p.bias_stride : static_cast<const T*>(p.weight);
-    const float braw = ld_uniform(br);
+    const float braw = ld_row<!SHORT>(br);
+    if constexpr (!SHORT) {
 #pragma unroll
-    for (int k = 0; k < W; ++k) asm volatile("" ::"s"(w[k]));
-    asm volatile("" ::"s"(braw), "s"(r.h), "s"(r.xn), "s"(r.gn));
-    __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0; k < W; ++k) asm volatile("" ::"s"(w[k]));
+        if constexpr (MODE != kRowsAny) asm volatile("" ::"s"(braw), "s"(r.h), "s"(r.xn), "s"(r.gn));
+        else asm volatile("" ::"s"(braw));
+        __builtin_amdgcn_sched_barrier(0);
+    }
     const float bias = p.bias ? braw : 0.0f;
-    // the pre-scaled weights are wave-uniform: kept in scalar registers
+    // the pre-scaled weights are wave-uniform (rows differ from lane to lane
+    // in kRowsShort alone): kept in scalar registers
     float wq[W];
 #pragma unroll
-    for (int k = 0; k < W; ++k) wq[k] = uniform_f32(-kLog2e * w[k]);
-    const float bq = uniform_f32(-kLog2e * bias);
-    if constexpr (SEQ) bwd_rows_compute_seq<T, W, VPT, SILU, FULL, RAG>(p, lane, b, c, t0, m, r, w, wq, bq, pw, pb);
-    else bwd_rows_compute<T, W, VPT, SILU, FULL, RAG>(p, lane, b, c, t0, m, r, w, wq, bq, pw, pb);
+    for (int k = 0; k < W; ++k) wq[k] = SHORT ? -kLog2e * w[k] : uniform_f32(-kLog2e * w[k]);
+    const float bq = SHORT ? -kLog2e * bias : uniform_f32(-kLog2e * bias);
+    if constexpr (SEQ)
+        bwd_rows_compute_seq<T, W, VPT, SILU, FULL, MODE>(p, lane, lastl, b, c, t0, L, m, r, w, wq, bq, pw, pb);
+    else
+        bwd_rows_compute<T, W, VPT, SILU, FULL, MODE>(p, lane, lastl, b, c, t0, L, m, r, w, wq, bq, pw, pb);
 }
 
 // One (row, segment) item per wavefront, kRowsWPB per block; item = (row,
@@ -627,7 +715,7 @@ __device__ __forceinline__ void bwd_rows_item(const cc1d_bwd_params& p, int lane
 // in LDS and written in the dtype, so the typed backward needs no second
 // launch -- measured 2 us slower at C2: the block's rows lie in B regions
 // of the tensors instead of one.)
-template <typename T, int W, int VPT, bool SILU, bool SEQ, bool RAG>
+template <typename T, int W, int VPT, bool SILU, bool SEQ, int MODE>
 __global__ void __launch_bounds__(64 * kRowsWPB) bwd_rows_vec(const BwdArgs a) {
     constexpr int SEG = 64 * VPT * elems16<T>::value;
     const cc1d_bwd_params& p = a.p;
@@ -644,20 +732,17 @@ __global__ void __launch_bounds__(64 * kRowsWPB) bwd_rows_vec(const BwdArgs a) {
 #pragma unroll
     for (int k = 0; k < W; ++k) pw[k] = 0.0f;
     float pb = 0.0f;
-    constexpr int EPV = elems16<T>::value;
-    // ragged rows: the row starts m elements past a 16-byte boundary
-    int32_t m = 0;
-    if constexpr (RAG) {
+    int32_t m = 0;  // the row starts m elements past a 16-byte boundary
+    if constexpr (MODE == kRowsAlike) {
         const T* xrow = static_cast<const T*>(p.x) + (int64_t)b * p.x_stride[0] + (int64_t)c * p.x_stride[1];
-        m = (int32_t)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(xrow) / sizeof(T)) & (EPV - 1));
+        m = (int32_t)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(xrow) / sizeof(T)) & (elems16<T>::value - 1));
     }
-    const int32_t Lv = (int32_t)p.seqlen + m;
-    // a ragged row's last segment may lie past its end: it adds nothing but
-    // still writes its (zero) record
-    if ((t0 > 0 || m == 0) && t0 + SEG <= Lv)
-        bwd_rows_item<T, W, VPT, SILU, SEQ, true, RAG>(p, lane, b, c, t0, m, pw, pb);
-    else if (!RAG || t0 < Lv)
-        bwd_rows_item<T, W, VPT, SILU, SEQ, false, RAG>(p, lane, b, c, t0, m, pw, pb);
+    const int32_t L = (int32_t)p.seqlen + m;
+    // a row may end before its last segment: that adds nothing but still writes its (zero) record
+    if ((t0 > 0 || m == 0) && t0 + SEG <= L)
+        bwd_rows_item<T, W, VPT, SILU, SEQ, true, MODE>(p, lane, 63, b, c, t0, L, m, pw, pb);
+    else if (MODE != kRowsAlike || t0 < L)
+        bwd_rows_item<T, W, VPT, SILU, SEQ, false, MODE>(p, lane, 63, b, c, t0, L, m, pw, pb);
 
     // ---- weight / bias gradient: wavefront sum, then lanes 0..W add ----
     float mine = wave_sum(pb);
@@ -673,6 +758,60 @@ __global__ void __launch_bounds__(64 * kRowsWPB) bwd_rows_vec(const BwdArgs a) {
     } else if (lane == W && p.dbias_acc != nullptr) {
         unsafeAtomicAdd(p.dbias_acc + (int64_t)c * p.dbias_acc_stride, mine);
     }
+}
+
+// Rows of nvec <= 32 vectors: a wavefront takes 64 / nvec (rounded down)
+// consecutive rows, lane l vector l % nvec of row l / nvec, neighbouring
+// lanes exchanging windows as in bwd_rows_vec but for a row's first and last
+// lane. The weight and bias sums of a row are added across its nvec lanes by
+// halving strides (ds_bpermute; a row's lanes are any run of lanes, so the
+// fixed DPP patterns do not fit), in the same order on every run.
+template <typename T, int W, bool SILU, bool SEQ>
+__global__ void __launch_bounds__(64 * kRowsWPB) bwd_rows_short(const BwdArgs a) {
+    const cc1d_bwd_params& p = a.p;
+    const uint32_t wl = threadIdx.x & 63;
+    const uint32_t nv = (uint32_t)a.nvec, per = (uint32_t)a.chunk;  // vectors per row, rows per wavefront
+    const uint32_t r = a.nseg_div.div(wl);
+    const uint32_t row0 = uniform32(blockIdx.x * (uint32_t)kRowsWPB + (threadIdx.x >> 6)) * per;
+    if (row0 >= (uint32_t)a.n_items) return;
+    const bool on = r < per && row0 + r < (uint32_t)a.n_items;
+    const uint32_t row = on ? row0 + r : row0;
+    const uint32_t b = a.dim_div.div(row);
+    const uint32_t c = row - b * (uint32_t)p.dim;
+    const int lane = (int)(wl - r * nv);  // vector of the row
+    float pw[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) pw[k] = 0.0f;
+    float pb = 0.0f;
+    bwd_rows_item<T, W, 1, SILU, SEQ, false, kRowsShort>(p, lane, (int)nv - 1, b, c, 0, on ? (int32_t)p.seqlen : 0,
+                                                         0, pw, pb);
+    // lane i of a row adds lane i + s while that lane is the row's, s = 16 .. 1
+#pragma unroll
+    for (int s = 16; s >= 1; s >>= 1) {
+        if ((uint32_t)s < nv) {  // wave-uniform
+            const bool add = lane < s && lane + s < (int)nv;
+            const int from = (int)(wl + s) & 63;
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                const float o = lane_get(pw[k], from);
+                pw[k] = add ? pw[k] + o : pw[k];
+            }
+            const float o = lane_get(pb, from);
+            pb = add ? pb + o : pb;
+        }
+    }
+    if (lane != 0 || !on) return;
+    if (a.part != nullptr) {  // record (W taps, bias) of this row
+        float* rec = a.part + (int64_t)row * (W + 1);
+#pragma unroll
+        for (int k = 0; k < W; ++k) rec[k] = pw[k];
+        rec[W] = pb;
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+        unsafeAtomicAdd(p.dweight_acc + (int64_t)c * p.dweight_acc_stride[0] + k * p.dweight_acc_stride[1], pw[k]);
+    if (p.dbias_acc != nullptr) unsafeAtomicAdd(p.dbias_acc + (int64_t)c * p.dbias_acc_stride, pb);
 }
 
 // One channel c of batch b over steps [t0, t1), any strides: writes dx (and
@@ -1289,20 +1428,15 @@ bool rows_vec_ok(const cc1d_bwd_params& p) {
     return true;
 }
 
-// ragged rows (a seqlen that is not a multiple of the vector, or rows that do
-// not start on a 16-byte boundary): unit time stride, and dout and dx laid out
-// like x modulo the vector -- the same element strides modulo EPV and bases a
-// multiple of 16 bytes apart -- so every row of each starts as far past a
-// 16-byte boundary as its row of x; seq_idx with a unit time stride
+// rows of any length at any element boundary: unit time stride is all they
+// need (seq_idx too, as 16-byte vectors of 4 ids are read from it)
 template <typename T>
-bool rows_ragged_ok(const cc1d_bwd_params& p) {
+bool rows_any_ok(const cc1d_bwd_params& p) {
     constexpr int64_t EPV = elems16<T>::value;
     if (p.width - 1 > EPV) return false;
     if (p.x_stride[2] != 1 || p.dout_stride[2] != 1 || p.dx_stride[2] != 1) return false;
-    for (const int64_t* s : {p.dout_stride, p.dx_stride})
-        if ((s[0] - p.x_stride[0]) % EPV != 0 || (s[1] - p.x_stride[1]) % EPV != 0) return false;
-    const intptr_t x = reinterpret_cast<intptr_t>(p.x);
-    if ((reinterpret_cast<intptr_t>(p.dout) - x) % 16 != 0 || (reinterpret_cast<intptr_t>(p.dx) - x) % 16 != 0)
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.dout) | reinterpret_cast<uintptr_t>(p.dx)) %
+        sizeof(T))
         return false;
     if (p.seq_idx != nullptr && (p.seq_idx_stride[1] != 1 || reinterpret_cast<uintptr_t>(p.seq_idx) % 4 != 0))
         return false;
@@ -1310,6 +1444,18 @@ bool rows_ragged_ok(const cc1d_bwd_params& p) {
     if (p.seqlen + 64 * 4 * EPV + EPV >= lim) return false;
     if (p.batch * p.dim * ceil_div(p.seqlen + EPV, 64 * EPV) >= lim) return false;
     return true;
+}
+
+// rows_any_ok, and dout and dx laid out like x modulo the vector: the same
+// element strides modulo EPV, bases a multiple of 16 bytes apart
+template <typename T>
+bool rows_alike(const cc1d_bwd_params& p) {
+    constexpr int64_t EPV = elems16<T>::value;
+    if (!rows_any_ok<T>(p)) return false;
+    for (const int64_t* s : {p.dout_stride, p.dx_stride})
+        if ((s[0] - p.x_stride[0]) % EPV != 0 || (s[1] - p.x_stride[1]) % EPV != 0) return false;
+    const intptr_t x = reinterpret_cast<intptr_t>(p.x);
+    return (reinterpret_cast<intptr_t>(p.dout) - x) % 16 == 0 && (reinterpret_cast<intptr_t>(p.dx) - x) % 16 == 0;
 }
 
 // channel-last tiles: unit channel stride, CPL | dim, rows aligned to the
@@ -1346,10 +1492,11 @@ bool cl_ok(const cc1d_bwd_params& p) {
 
 enum BwdKind { kBwdRows = 0, kBwdCl = 1, kBwdGeneric = 2 };
 
-// Kernel choice and launch geometry for one call; shared by the launch, the
-// workspace size and the partial-sum reduction.
+// Kernel choice and launch geometry for one call; shared by the launch and
+// the partial-sum reduction.
 struct BwdPlan {
     int kind;
+    int mode;          // rows: RowsMode
     int vpt;           // rows: 16-byte vectors per lane
     int cpl;           // cl: channels per lane
     BwdArgs a;
@@ -1357,6 +1504,20 @@ struct BwdPlan {
     int64_t records;   // partial-sum records (rows / generic: items; cl: blocks)
     int64_t rec_floats;
 };
+
+// Vectors per lane of a row of nvec vectors (measured at C2's batch and dim):
+// 4 from 129 vectors a row on -- one segment of 4 beats two of 2, the same
+// lane slots (L = 1536: 38.8 instead of 45.2 us), when the grid keeps 2048
+// wavefronts (on smaller grids the more wavefronts of 2 measured faster) --
+// except when a row a little longer than a multiple of the 4-vector segment
+// would leave its last one mostly empty: 2 when that takes at most 85 % of
+// the lane slots (L = 2056: 58.8 instead of 65.7 us; 4104: 99.8 instead of 105.2)
+inline int rows_vpt(int64_t nvec, int64_t rows) {
+    const int64_t per = ceil_div(nvec, 64);
+    int vpt = per >= 4 || (per == 3 && rows >= 2048) ? 4 : (per >= 2 ? 2 : 1);
+    if (vpt == 4 && ceil_div(nvec, 128) * 128 * 100 <= ceil_div(nvec, 256) * 256 * 85) vpt = 2;
+    return vpt;
+}
 
 template <typename T, int W>
 BwdPlan plan_bwd(const cc1d_bwd_params& p) {
@@ -1366,33 +1527,51 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
     pl.a.part = nullptr;
     pl.a.chunk = 0;
     pl.a.groups = 0;
+    pl.a.nvec = 0;
+    pl.mode = kRowsAligned;
     pl.vpt = 0;
     pl.cpl = 0;
     pl.rec_floats = W + 1;
-    pl.a.ragged = 0;
     const bool aligned = W - 1 <= EPV && rows_vec_ok<T>(p);
-    if (aligned || (W - 1 <= EPV && rows_ragged_ok<T>(p))) {
-        pl.a.ragged = aligned ? 0 : 1;
-        // vectors a row spans: a ragged row may start up to EPV - 1 elements
-        // past a vector boundary
-        const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
-        const int64_t per = ceil_div(nvec, 64);
-        pl.kind = kBwdRows;
-        // vectors per lane (measured at C2's batch and dim): 4 from 129 vectors
-        // a row on -- one segment of 4 beats two of 2, the same lane slots
-        // (L = 1536: 38.8 instead of 45.2 us), when the grid keeps 2048
-        // wavefronts (on smaller grids the more wavefronts of 2 measured faster)
-        // -- except when a row a little longer
-        // than a multiple of the 4-vector segment would leave its last one
-        // mostly empty: 2 when that takes at most 85 % of the lane slots
-        // (L = 2056: 58.8 instead of 65.7 us; 4104: 99.8 instead of 105.2)
+    if (aligned || (W - 1 <= EPV && rows_any_ok<T>(p))) {
+        const int64_t least = ceil_div(p.seqlen, EPV);  // vectors from the row's first element on
         const int64_t rows = p.batch * p.dim;
-        pl.vpt = per >= 4 || (per == 3 && rows >= 2048) ? 4 : (per >= 2 ? 2 : 1);
-        if (pl.vpt == 4 && ceil_div(nvec, 128) * 128 * 100 <= ceil_div(nvec, 256) * 256 * 85) pl.vpt = 2;
-        pl.a.nseg = ceil_div(nvec, 64 * (int64_t)pl.vpt);
-        pl.a.n_items = p.batch * p.dim * pl.a.nseg;
-        pl.a.nseg_div = FastDiv((uint32_t)pl.a.nseg);
+        pl.kind = kBwdRows;
         pl.a.dim_div = FastDiv((uint32_t)p.dim);
+        if (least <= kShortVecs && rows_any_ok<T>(p)) {
+            pl.mode = kRowsShort;
+            pl.vpt = 1;
+            pl.a.nvec = (int32_t)least;
+            pl.a.chunk = 64 / least;
+            pl.a.nseg = 1;
+            pl.a.n_items = rows;
+            pl.a.nseg_div = FastDiv((uint32_t)least);
+            pl.blocks = ceil_div(ceil_div(rows, pl.a.chunk), (int64_t)kRowsWPB);
+            pl.records = rows;
+            return pl;
+        }
+        pl.mode = aligned ? kRowsAligned : kRowsAny;
+        pl.vpt = rows_vpt(least, rows);
+        pl.a.nseg = ceil_div(least, 64 * (int64_t)pl.vpt);
+        if (!aligned && rows_alike<T>(p)) {
+            // a row that starts past a vector boundary may span one more
+            const int64_t nvec = ceil_div(p.seqlen + EPV - 1, EPV);
+            const int vpt = rows_vpt(nvec, rows);
+            const int64_t nseg = ceil_div(nvec, 64 * (int64_t)vpt);
+            // aligned vectors, unless that one more costs over 15 % of the lane slots
+            // (16-bit types, us at C2's batch and dim, aligned -> unaligned: L = 2047
+            // 60.9 -> 50.0, 1023 40.1 -> 28.0, 511 23.8 -> 18.7; at ten times the batch
+            // 575 -> 456, 350 -> 242, 191 -> 146). Otherwise alignment wins: unaligned
+            // stores cost 7-20 % of a large fp32 or long-row call (fp32, batch 40,
+            // L = 2047: 850 -> 928; bf16 8 x 2048 x 16383: 272 -> 335).
+            if (sizeof(T) == 4 || pl.vpt * pl.a.nseg * 100 > vpt * nseg * 85) {
+                pl.mode = kRowsAlike;
+                pl.vpt = vpt;
+                pl.a.nseg = nseg;
+            }
+        }
+        pl.a.n_items = rows * pl.a.nseg;
+        pl.a.nseg_div = FastDiv((uint32_t)pl.a.nseg);
         pl.blocks = ceil_div(pl.a.n_items, (int64_t)kRowsWPB);
         pl.records = pl.a.n_items;
         return pl;
@@ -1424,12 +1603,33 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
         return pl;
     }
     pl.kind = kBwdGeneric;
-    pl.a.chunk = 64;
+    pl.a.chunk = kGenericChunk;
     pl.a.nseg = ceil_div(p.seqlen, pl.a.chunk);
     pl.a.n_items = p.batch * p.dim * pl.a.nseg;
     pl.blocks = ceil_div(pl.a.n_items, 256);
     pl.records = pl.a.n_items;
     return pl;
+}
+
+// The workspace of a call: what cc1d_bwd_workspace_floats tells the caller and
+// cc1d_bwd_typed asks for. For rows it depends on sizes and layout alone and
+// not on the launch geometry -- segments of the vectors that a row spans, or
+// time chunks where the tensors lie unlike each other -- so that a size a
+// program has stored, or a problem that fits the static scratch, stays good
+// when a kernel splits rows another way. Every plan's records fit: kRowsShort
+// has one per row, kRowsAny at most one per 64 steps.
+template <typename T, int W>
+int64_t reserved_floats(const cc1d_bwd_params& p, const BwdPlan& pl) {
+    if (pl.kind != kBwdRows || pl.mode == kRowsAligned || pl.mode == kRowsAlike) return pl.records * pl.rec_floats;
+    constexpr int64_t EPV = elems16<T>::value;
+    const int64_t rows = p.batch * p.dim;
+    const bool aligned = rows_vec_ok<T>(p);
+    int64_t n = ceil_div(p.seqlen, (int64_t)kGenericChunk);
+    if (aligned || rows_alike<T>(p)) {
+        const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
+        n = ceil_div(nvec, 64 * (int64_t)rows_vpt(nvec, rows));
+    }
+    return rows * n * pl.rec_floats;
 }
 
 template <typename T, int W, bool SILU>
@@ -1441,12 +1641,16 @@ int launch_plan(const BwdPlan& pl, const cc1d_bwd_params& p, hipStream_t stream)
             return with_flag(p.seq_idx != nullptr, [&](auto qc) {
                 constexpr bool SEQ = decltype(qc)::value;
                 const dim3 block(64 * kRowsWPB);
-                return with_flag(a.ragged != 0, [&](auto rc) {
-                    constexpr bool RAG = decltype(rc)::value;
-                    if (pl.vpt == 4) return launch(bwd_rows_vec<T, W, 4, SILU, SEQ, RAG>, grid, block, stream, a);
-                    if (pl.vpt == 2) return launch(bwd_rows_vec<T, W, 2, SILU, SEQ, RAG>, grid, block, stream, a);
-                    return launch(bwd_rows_vec<T, W, 1, SILU, SEQ, RAG>, grid, block, stream, a);
-                });
+                if (pl.mode == kRowsShort) return launch(bwd_rows_short<T, W, SILU, SEQ>, grid, block, stream, a);
+                auto go = [&](auto mc) {
+                    constexpr int MODE = decltype(mc)::value;
+                    if (pl.vpt == 4) return launch(bwd_rows_vec<T, W, 4, SILU, SEQ, MODE>, grid, block, stream, a);
+                    if (pl.vpt == 2) return launch(bwd_rows_vec<T, W, 2, SILU, SEQ, MODE>, grid, block, stream, a);
+                    return launch(bwd_rows_vec<T, W, 1, SILU, SEQ, MODE>, grid, block, stream, a);
+                };
+                if (pl.mode == kRowsAligned) return go(std::integral_constant<int, kRowsAligned>{});
+                if (pl.mode == kRowsAlike) return go(std::integral_constant<int, kRowsAlike>{});
+                return go(std::integral_constant<int, kRowsAny>{});
             });
         }
         return CC1D_ERR_SHAPE;  // not reached: the plan only picks rows when the halo fits
@@ -1607,8 +1811,8 @@ template <typename T>
 int64_t bwd_workspace_floats_dtype(const cc1d_bwd_params& p) {
     int64_t n = -1;
     with_width(p.width, [&](auto wc) {
-        const BwdPlan pl = plan_bwd<T, decltype(wc)::value>(p);
-        n = pl.records * pl.rec_floats;
+        constexpr int W = decltype(wc)::value;
+        n = reserved_floats<T, W>(p, plan_bwd<T, W>(p));
         return (int)CC1D_OK;
     });
     return n;
@@ -1620,7 +1824,7 @@ int launch_bwd_typed_dtype(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hi
         constexpr int W = decltype(wc)::value;
         return with_flag(p.apply_silu != 0, [&](auto sc) {
             BwdPlan pl = plan_bwd<T, W>(p);
-            if (pl.records * pl.rec_floats > g.workspace_floats) return (int)CC1D_ERR_WORKSPACE;
+            if (reserved_floats<T, W>(p, pl) > g.workspace_floats) return (int)CC1D_ERR_WORKSPACE;
             if (g.workspace == nullptr) return (int)CC1D_ERR_NULL_POINTER;
             pl.a.part = g.workspace;
             const int st = launch_plan<T, W, decltype(sc)::value>(pl, p, stream);

@@ -106,6 +106,76 @@ template <typename T> __device__ __forceinline__ void vstore_nt(T* p, const u32x
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// The same 16-byte accesses at any element boundary. The hardware takes a
+// dwordx4 at any 2-byte address (the HSA ABI turns unaligned access on), in
+// one instruction: copying 20480 rows of 4 KB takes 27.6 us from and to
+// aligned addresses, 29.4 with the loads one bf16 off, 30.0 with the stores,
+// 31.3 with both, and 30.1 with rows of 2041 elements (every offset occurs).
+template <int BYTES> struct AnyAddr;  // dword types at element boundaries
+template <> struct AnyAddr<2> {
+    typedef u32x4 __attribute__((aligned(2))) v4;
+    typedef u32x2 __attribute__((aligned(2))) v2;
+    typedef uint32_t __attribute__((aligned(2))) v1;
+};
+template <> struct AnyAddr<4> {
+    typedef u32x4 __attribute__((aligned(4))) v4;
+    typedef u32x2 __attribute__((aligned(4))) v2;
+    typedef uint32_t v1;
+};
+template <typename T> __device__ __forceinline__ u32x4 vload_any(const T* p) {
+    return *reinterpret_cast<const typename AnyAddr<sizeof(T)>::v4*>(p);
+}
+template <typename T> __device__ __forceinline__ u32x4 vload_any_nt(const T* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const typename AnyAddr<sizeof(T)>::v4*>(p));
+}
+template <typename T> __device__ __forceinline__ void vstore_any_nt(T* p, const u32x4& v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<typename AnyAddr<sizeof(T)>::v4*>(p));
+}
+
+// The first rem (1 .. EPV - 1, the same for every lane) elements of a 16-byte
+// vector at p: a row's last ones, where reading the whole vector would leave
+// the row. Read as at most one access each of 8, 4 and 2 bytes; load() only
+// issues them, vec() waits and puts them in place (zero from rem on), so a
+// kernel can issue its other loads in between.
+template <typename T> struct RowTail {
+    u32x2 a;
+    uint32_t b, c;
+    __device__ __forceinline__ void load(const T* p, int rem) {
+        typedef typename AnyAddr<sizeof(T)>::v2 any2;
+        typedef typename AnyAddr<sizeof(T)>::v1 any1;
+        constexpr int PER = 4 / (int)sizeof(T);  // elements per dword
+        a = u32x2{0u, 0u};
+        b = c = 0u;
+        if (rem & (2 * PER)) a = *reinterpret_cast<const any2*>(p);
+        if (rem & PER) b = *reinterpret_cast<const any1*>(p + (rem & (2 * PER)));
+        if constexpr (PER == 2) {
+            if (rem & 1) c = *reinterpret_cast<const uint16_t*>(p + (rem & 6));
+        }
+    }
+    __device__ __forceinline__ u32x4 vec(int rem) const {
+        constexpr int PER = 4 / (int)sizeof(T);
+        const bool two = (rem & (2 * PER)) != 0, one = (rem & PER) != 0;
+        u32x4 r;
+        r[0] = two ? a[0] : (one ? b : c);
+        r[1] = two ? a[1] : (one ? c : 0u);
+        r[2] = two ? (one ? b : c) : 0u;
+        r[3] = two && one ? c : 0u;
+        return r;
+    }
+    // the first rem elements of v to p
+    static __device__ __forceinline__ void store(T* p, const u32x4& v, int rem) {
+        typedef typename AnyAddr<sizeof(T)>::v2 any2;
+        typedef typename AnyAddr<sizeof(T)>::v1 any1;
+        constexpr int PER = 4 / (int)sizeof(T);
+        const bool two = (rem & (2 * PER)) != 0, one = (rem & PER) != 0;
+        if (two) *reinterpret_cast<any2*>(p) = u32x2{v[0], v[1]};
+        if (one) *reinterpret_cast<any1*>(p + (rem & (2 * PER))) = two ? v[2] : v[0];
+        if constexpr (PER == 2) {
+            if (rem & 1) *reinterpret_cast<uint16_t*>(p + (rem & 6)) = (uint16_t)(two ? (one ? v[3] : v[2]) : (one ? v[1] : v[0]));
+        }
+    }
+};
+
 // N consecutive elements of T held as raw dwords, N * sizeof(T) in {4, 8, 16}
 // (one global_load / store of 1, 2 or 4 dwords per lane). Element indices
 // are compile-time after unrolling.
@@ -206,15 +276,22 @@ template <typename T> __device__ __forceinline__ uint32_t lead_mask(int d, int32
     if constexpr (sizeof(T) == 4) return d < n ? ~0u : 0u;
     else return 2 * d + 1 < n ? ~0u : (2 * d < n ? 0xffffu : 0u);
 }
-// Storage bits of an fp32 value that T represents exactly.
-template <typename T> __device__ __forceinline__ uint32_t tbits(float v) {
-    if constexpr (sizeof(T) == 4) return __float_as_uint(v);
-    else return from_f32<T>(v).bits;
-}
 // Store element e of the packed vector v at p (its raw bits: no rounding).
 template <typename T> __device__ __forceinline__ void st_elem(T* p, const u32x4& v, int e) {
     if constexpr (sizeof(T) == 4) *reinterpret_cast<uint32_t*>(p) = v[e];
     else *reinterpret_cast<uint16_t*>(p) = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+}
+// Elements m .. EPV - 1 (m > 0, the same for every lane) of v to p + m ..
+template <typename T> __device__ __forceinline__ void store_from(T* p, const u32x4& v, int m) {
+#pragma unroll
+    for (int e = 1; e < elems16<T>::value; ++e) {
+        if (e >= m) st_elem<T>(p + e, v, e);
+    }
+}
+// Storage bits of an fp32 value that T represents exactly.
+template <typename T> __device__ __forceinline__ uint32_t tbits(float v) {
+    if constexpr (sizeof(T) == 4) return __float_as_uint(v);
+    else return from_f32<T>(v).bits;
 }
 
 // a[k] for a runtime k (0 outside [0, N)), as a chain of selects: a register
@@ -225,6 +302,21 @@ template <int N> __device__ __forceinline__ float pick(const float* a, int k) {
     for (int i = 0; i < N; ++i) r = (i == k) ? a[i] : r;
     return r;
 }
+
+// How a wavefront of the row kernels takes rows whose time stride is one.
+//   kRowsAligned  one row, on 16-byte boundaries, whole vectors long
+//   kRowsAlike    one row of any start and length that lies alike in every
+//                 tensor modulo 16 bytes: vectors count from the boundary at
+//                 or before the row's first element, so every access is
+//                 aligned (a vector that holds one of the row's elements is in
+//                 the same memory page, so reading it whole is safe)
+//   kRowsAny      one row of any start and length, wherever it lies in each
+//                 tensor: unaligned vectors from its first element on
+//   kRowsShort    several rows of at most 32 vectors, read as in kRowsAny, one
+//                 vector per lane: the row and all that belongs to it differ
+//                 from lane to lane
+enum RowsMode { kRowsAligned = 0, kRowsAlike = 1, kRowsAny = 2, kRowsShort = 3 };
+constexpr int64_t kShortVecs = 32;  // vectors of the longest row of kRowsShort
 
 // Wavefront-uniform value (lets the compiler keep it in an SGPR).
 __device__ __forceinline__ uint32_t uniform32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -245,61 +337,21 @@ __device__ __forceinline__ int32_t opaque(int32_t v) {
     return v;
 }
 
-// The N (4 or 8) ids of row positions pos .. pos + N - 1 of one seq_idx row
-// (sr, L ids, unit stride; -1 outside [0, L)), read as the N/4 + 1 aligned
-// 16-byte vectors that cover them (ids_load) and shifted into place
-// (ids_shift): r = the first id's offset in its vector (the same for every
-// lane), a0 = sr's own offset in its vector. MASK: some position may lie
-// outside the row; a lane with none inside loads nothing, and a vector that
-// holds none of the row's ids reads the row's first vector instead, as does
-// the last one when r == 0 (not needed then), so every access stays inside
-// the row's allocation. A kernel issues every vector's loads before the
-// first shift: a shift right behind its loads waits for them, before the
-// next vector's loads are issued.
-template <int N> struct IdsRaw {
-    u32x4 v[N / 4 + 1];
-};
-
-template <int N, bool MASK>
-__device__ __forceinline__ void ids_load(const int32_t* sr, int32_t L, int32_t pos, int r, int a0, IdsRaw<N>& raw) {
-    static_assert(N == 4 || N == 8, "one or two 16-byte vectors");
-    constexpr int NV = N / 4 + 1;
-    const int32_t q0 = pos - r;  // first row position of the first vector (16-byte aligned)
-    if (!MASK || (pos + N > 0 && pos < L)) {
+// The ids of the N (4 or 8) row positions from p on, at any 4-byte address.
+template <int N> __device__ __forceinline__ void ids_any(const int32_t* p, int32_t* id) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            int32_t q = q0 + 4 * v;
-            if (v == NV - 1) q = r != 0 ? q : q0;
-            if constexpr (MASK) q = (q + 3 >= 0 && q < L) ? q : -a0;
-            raw.v[v] = *reinterpret_cast<const u32x4*>(sr + q);
-        }
-    } else {
+    for (int q = 0; q < N / 4; ++q) {
+        const u32x4 s = *reinterpret_cast<const AnyAddr<4>::v4*>(p + 4 * q);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) raw.v[v] = vzero();  // masked to -1 by ids_shift
+        for (int r = 0; r < 4; ++r) id[4 * q + r] = (int32_t)s[r];
     }
 }
-
-// The shift is two levels of v_perm_b32 (one dword of two, by the bits of
-// r): selects on a scalar r became branches, each waiting for its loads, and
-// selects on a vector-register r an indexed copy through scratch memory.
-template <int N, bool MASK>
-__device__ __forceinline__ void ids_shift(const IdsRaw<N>& raw, int32_t L, int32_t pos, int r, int32_t* out) {
-    uint32_t c[N + 4];
+// ids from .. to - 1 (the same range for every lane) of the N from p on,
+// element by element; the others keep what id holds.
+template <int N> __device__ __forceinline__ void ids_some(const int32_t* p, int from, int to, int32_t* id) {
 #pragma unroll
-    for (int v = 0; v < N / 4 + 1; ++v)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) c[4 * v + i] = raw.v[v][i];
-    // byte selectors of v_perm_b32(hi, lo, sel): 0x07060504 picks hi, 0x03020100 lo
-    const uint32_t s2 = (r & 2) ? 0x07060504u : 0x03020100u;
-    const uint32_t s1 = (r & 1) ? 0x07060504u : 0x03020100u;
-    uint32_t t[N + 2];
-#pragma unroll
-    for (int e = 0; e < N + 2; ++e) t[e] = __builtin_amdgcn_perm(c[e + 2], c[e], s2);
-#pragma unroll
-    for (int e = 0; e < N; ++e) {
-        out[e] = (int32_t)__builtin_amdgcn_perm(t[e + 1], t[e], s1);
-        if constexpr (MASK) out[e] = (pos + e >= 0 && pos + e < L) ? out[e] : -1;
-    }
+    for (int e = 0; e < N; ++e)
+        if (e >= from && e < to) id[e] = p[e];
 }
 
 // SiLU = x * sigmoid(x), as x * rcp(1 + exp(-x)) in fp32.

@@ -15,13 +15,13 @@
 //                    halo before a vector comes from the neighbouring lane
 //                    (ds_bpermute); only lane 0 of a segment reads one extra
 //                    vector from global memory. No LDS, no barriers.
-//                    Ragged rows (a start that is not 16-byte aligned, or a
-//                    length that is not a multiple of the vector) are read in
-//                    the 16-byte vectors of their own memory: a row that starts
-//                    m elements past a vector boundary is walked from that
-//                    boundary, its first m elements (the previous row's) are
-//                    replaced by initial_states or zero, and the vectors it
-//                    shares with its neighbours are stored element by element.
+//                    Rows that are not whole aligned vectors (any start, any
+//                    length) are walked in the aligned vectors of their own
+//                    memory where out lies like x, else in unaligned ones
+//                    (RowsMode in cc1d_device.hpp); a row's first and last
+//                    few elements are stored in smaller pieces.
+//   fwd_rows_short -- rows of at most 32 vectors: a wavefront takes as many
+//                    whole rows as fit into its 64 lanes, a lane one vector.
 //   fwd_cl        -- rows contiguous along channels (channel-last). A lane owns
 //                    4 bytes of adjacent channels, a wavefront a tile of 16
 //                    time steps (plus W-1 halo rows) of 64 lanes' channels,
@@ -35,55 +35,69 @@ namespace cc1d {
 
 struct FwdArgs {
     cc1d_fwd_params p;
-    int32_t ragged;    // rows_vec: rows may start off a 16-byte boundary / end inside a vector (kernel variant)
-    FastDiv nseg_div;  // rows_vec: item -> row
+    FastDiv nseg_div;  // rows_vec: item -> row; rows_short: lane -> row of the wavefront
     FastDiv dim_div;   // rows_vec: row -> batch entry
-    int64_t nseg;     // segments (rows_vec), tiles (cl) or chunks (generic) per row
-    int64_t n_items;  // work items: segments / tiles / threads
-    int64_t chunk;    // time steps per item (cl / generic)
+    int64_t nseg;     // segments (rows_vec), tiles (cl) or chunks (generic) per row; rows_short: vectors per row
+    int64_t n_items;  // work items: segments / tiles / threads; rows_short: rows
+    int64_t chunk;    // time steps per item (cl / generic); rows_short: rows per wavefront
     int64_t ngroups;  // channel groups (cl)
 };
 
-// One wavefront-segment of one row. FULL: the whole segment lies inside the
-// row (no per-vector bounds checks).
-//
-// Positions t here count from the 16-byte boundary at or before the row's
-// first element: the row holds t in [m, m + L) (m = 0 for an aligned row), so
-// every vector access is aligned. A 16-byte vector that holds one of the
-// row's elements lies in the same memory page, so reading it whole is safe.
-template <typename T, int W, int VPT, bool SILU, bool SEQ, bool FULL, bool RAG>
+// One wavefront-segment of one row. Positions t count from m elements before
+// the row's first: the row is [m, m + L), m 0 except in kRowsAlike. FULL: the
+// whole segment lies inside the row (no per-vector bounds checks). on: the
+// lane has a row (kRowsShort; `lane` is then the lane's vector of its row).
+template <typename T, int W, int VPT, bool SILU, bool SEQ, bool FULL, int MODE>
 __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int lane, int64_t b, int64_t c,
-                                                 int32_t t0, int32_t m) {
+                                                 int32_t t0, int32_t m, bool on) {
     constexpr int EPV = elems16<T>::value;
     constexpr int H = W - 1;
-    const int32_t L = (int32_t)p.seqlen;
-    const int32_t Lv = L + m;  // end of the row
+    constexpr bool SHORT = MODE == kRowsShort, ALIKE = MODE == kRowsAlike;
+    constexpr bool ANY = MODE == kRowsAny || SHORT;  // unaligned vectors
+    static_assert(!SHORT || (VPT == 1 && !FULL), "short rows: one vector per lane");
+    const int32_t Le = (int32_t)p.seqlen + m;      // end of the row
+    const int32_t L = SHORT ? (on ? Le : 0) : Le;  // a lane without a row touches nothing
     const T* __restrict__ xr = static_cast<const T*>(p.x) + b * p.x_stride[0] + c * p.x_stride[1] - m;
     T* __restrict__ orow = static_cast<T*>(p.out) + b * p.out_stride[0] + c * p.out_stride[1] - m;
+
+    // the row's last rem elements are part of a vector, which starts at tp:
+    // vector jt of the lane with `tail`
+    constexpr bool EDGES = MODE != kRowsAligned && !FULL;
+    const int rem = EDGES ? Le & (EPV - 1) : 0;
+    const int32_t tp = Le - rem;
+    const int jt = SHORT ? 0 : (tp - t0) / (64 * EPV);
+    const bool tail = EDGES && rem != 0 && tp >= t0 && tp == t0 + (jt * 64 + lane) * EPV && on;
+    const bool head = ALIKE && !FULL && m > 0 && t0 == 0;  // wave-uniform: lane 0's first vector starts before the row
+    auto whole = [&](int32_t t) {  // the vector at t lies inside the row
+        return FULL || (MODE == kRowsAligned ? t < L : ALIKE ? t >= m && t + EPV <= L : t + EPV <= L);
+    };
 
     u32x4 v[VPT];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int32_t t = t0 + (j * 64 + lane) * EPV;
-        v[j] = (FULL || t < Lv) ? vload_nt(xr + t) : vzero();
+        if constexpr (ANY) v[j] = whole(t) ? vload_any_nt(xr + t) : vzero();
+        else v[j] = (FULL || t < L) ? vload_nt(xr + t) : vzero();
+    }
+    RowTail<T> xt;
+    if constexpr (ANY) {
+        xt.a = u32x2{0u, 0u};
+        xt.b = xt.c = 0u;
+        if (tail) xt.load(xr + tp, rem);
     }
     u32x4 h = vzero();
-    if (lane == 0 && t0 > 0) h = vload(xr - EPV + t0);
+    if constexpr (!SHORT) {
+        if (lane == 0 && t0 > 0) h = ANY ? vload_any(xr - EPV + t0) : vload(xr - EPV + t0);
+    }
 
     int32_t id[VPT][EPV];
     int32_t hid[H];
     if constexpr (SEQ) {
-        const int32_t* __restrict__ sr = p.seq_idx + b * p.seq_idx_stride[0];  // unit time stride
-        // ragged rows: a vector's ids start rid ids past a 16-byte boundary
-        // (its first position, t - m, is a multiple of 4 plus -m); the row's
-        // first id a0 past one
-        const int a0 = RAG ? (int)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(sr) / 4) & 3u) : 0;
-        const int rid = (a0 - m) & 3;
-        IdsRaw<EPV> raw[RAG ? VPT : 1];
+        const int32_t* __restrict__ sr = p.seq_idx + b * p.seq_idx_stride[0] - m;  // unit time stride
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
             const int32_t t = t0 + (j * 64 + lane) * EPV;
-            if constexpr (!RAG) {  // aligned rows: 16-byte vectors of 4 ids
+            if constexpr (MODE == kRowsAligned) {  // 16-byte vectors of 4 ids
 #pragma unroll
                 for (int q = 0; q < EPV / 4; ++q) {
                     const u32x4 s = (FULL || t < L) ? *reinterpret_cast<const u32x4*>(sr + t + 4 * q)
@@ -92,22 +106,23 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
                     for (int r = 0; r < 4; ++r) id[j][4 * q + r] = (int32_t)s[r];
                 }
             } else {
-                ids_load<EPV, !FULL>(sr, L, t - m, rid, a0, raw[j]);
-            }
-        }
-        if constexpr (RAG) {  // -1 outside the row
 #pragma unroll
-            for (int j = 0; j < VPT; ++j) {
-                const int32_t pos = t0 + (j * 64 + lane) * EPV - m;
-                const int32_t vs = t0 + j * 64 * EPV;  // vector j of lane 0: inside the row in every lane?
-                if (FULL || (vs >= m && vs + 64 * EPV <= Lv)) ids_shift<EPV, false>(raw[j], L, pos, rid, id[j]);
-                else ids_shift<EPV, true>(raw[j], L, pos, rid, id[j]);
+                for (int e = 0; e < EPV; ++e) id[j][e] = -1;
+                if (whole(t)) ids_any<EPV>(sr + t, id[j]);
+                // a row's first and last few ids, each into its own register (no
+                // wait here); wave-uniform tests around
+                if (EDGES && j == 0 && head) {
+                    if (lane == 0) ids_some<EPV>(sr, m, EPV, id[0]);
+                }
+                if (EDGES && j == jt && rem != 0) {
+                    if (tail) ids_some<EPV>(sr + t, 0, rem, id[j]);
+                }
             }
         }
 #pragma unroll
         for (int i = 0; i < H; ++i) {
-            const int32_t pos = t0 - H + i - m;
-            hid[i] = (lane == 0 && pos >= 0) ? sr[pos] : -1;
+            const int32_t pos = t0 - H + i;
+            hid[i] = (!SHORT && lane == 0 && pos >= m) ? sr[pos] : -1;
         }
     }
 
@@ -117,7 +132,7 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
     for (int k = 0; k < W; ++k) w[k] = ld(wr, k * p.weight_stride[1]);
     const float bias = p.bias ? ld(static_cast<const T*>(p.bias), c * p.bias_stride) : 0.0f;
 
-    const bool use_init = p.initial_states != nullptr && t0 == 0 && lane == 0;
+    const bool use_init = p.initial_states != nullptr && t0 == 0 && lane == 0 && on;
     float hinit[H];
 #pragma unroll
     for (int i = 0; i < H; ++i) {
@@ -127,36 +142,42 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
                           b * p.initial_states_stride[0] + c * p.initial_states_stride[1] +
                               i * p.initial_states_stride[2]);
     }
-    // the row's first vector holds m elements of the previous row: they are
-    // positions -m .. -1 of this one (initial_states or zero)
-    if (RAG && !FULL && t0 == 0 && m > 0 && lane == 0) {
+    // the first vector's m elements before the row (the previous row's) are
+    // positions -m .. -1 of this one: initial_states or zero
+    if (head && lane == 0) {
         float f[EPV];
 #pragma unroll
         for (int e = 0; e < EPV; ++e)  // initial_states slot e - m + H (none when negative)
             f[e] = e >= m ? vget<T>(v[0], e) : pick<H>(hinit, e - m + H);
         v[0] = vpack<T>(f);
     }
+    if (ANY && EDGES && rem != 0) {  // wave-uniform
+        const u32x4 tv = xt.vec(rem);  // zero in the lanes without the tail
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+            if (j == jt) v[j] |= tv;
+    }
 
     constexpr int D0 = ((EPV - H) * (int)sizeof(T)) / 4;  // first dword of the needed tail
-    const int prev_lane = (lane + 63) & 63;
+    const int wl = SHORT ? (int)(threadIdx.x & 63) : lane;  // lane of the wavefront
+    const int prev_lane = (wl + 63) & 63;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int32_t t = t0 + (j * 64 + lane) * EPV;
         u32x4 pv = vzero();
 #pragma unroll
         for (int d = D0; d < 4; ++d) {
-            const uint32_t send = (lane == 63) ? (j > 0 ? v[j > 0 ? j - 1 : 0][d] : 0u) : v[j][d];
+            const uint32_t send = (!SHORT && lane == 63) ? (j > 0 ? v[j > 0 ? j - 1 : 0][d] : 0u) : v[j][d];
             pv[d] = lane_get(send, prev_lane);
         }
         if (j == 0 && lane == 0) pv = h;
         float win[H + EPV];
-        // before the row (t0 == 0, lane 0): position i - H - m, initial_states slot i - m
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-            if constexpr (FULL || !RAG)  // m == 0 whenever a first segment is full
-                win[i] = (j == 0 && use_init) ? hinit[i] : vget<T>(pv, EPV - H + i);
-            else
+        for (int i = 0; i < H; ++i) {  // before the row: position i - H, initial_states slot i - m
+            if constexpr (ALIKE && !FULL)
                 win[i] = (j == 0 && use_init) ? pick<H>(hinit, i - m) : vget<T>(pv, EPV - H + i);
+            else  // m == 0 whenever a first segment is full
+                win[i] = (j == 0 && use_init) ? hinit[i] : vget<T>(pv, EPV - H + i);
         }
 #pragma unroll
         for (int i = 0; i < EPV; ++i) win[H + i] = vget<T>(v[j], i);
@@ -165,8 +186,8 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
         if constexpr (SEQ) {
 #pragma unroll
             for (int i = 0; i < H; ++i) {
-                const int32_t send = (lane == 63) ? (j > 0 ? id[j > 0 ? j - 1 : 0][EPV - H + i] : -1)
-                                                  : id[j][EPV - H + i];
+                const int32_t send = (!SHORT && lane == 63) ? (j > 0 ? id[j > 0 ? j - 1 : 0][EPV - H + i] : -1)
+                                                            : id[j][EPV - H + i];
                 const int32_t r = lane_get(send, prev_lane);
                 sw[i] = (j == 0 && lane == 0) ? hid[i] : r;
             }
@@ -186,29 +207,28 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
             }
             o[i] = acc;
         }
-        if constexpr (!RAG) {
-            if (FULL || t < L) vstore_nt(orow + t, vpack<T>(o));
-        } else {
-            const u32x4 ov = vpack<T>(o);
-            if (FULL || (t >= m && t + EPV <= Lv)) {
-                vstore_nt(orow + t, ov);
-            } else if (t < Lv) {  // a vector shared with a neighbouring row
-#pragma unroll
-                for (int e = 0; e < EPV; ++e)
-                    if ((uint32_t)(t + e - m) < (uint32_t)(Lv - m)) st_elem<T>(orow + t + e, ov, e);
-            }
+        const u32x4 ov = vpack<T>(o);
+        if (whole(t)) {
+            if constexpr (ANY) vstore_any_nt(orow + t, ov);
+            else vstore_nt(orow + t, ov);
+        }
+        if (EDGES && j == 0 && head) {
+            if (lane == 0) store_from(orow, ov, m);
+        }
+        if (EDGES && j == jt && rem != 0) {  // wave-uniform
+            if (tail) RowTail<T>::store(orow + t, ov, rem);
         }
 
         // final_states (_fn.py:31-50): the lane holding the row's last
         // position writes the last W-1 columns from its window (they are
         // positions t - H .. t + EPV - 1)
-        if (p.final_states_out != nullptr && (RAG ? (t < Lv && Lv <= t + EPV) : t + EPV == L)) {
+        if (p.final_states_out != nullptr && (MODE != kRowsAligned ? (t < L && L <= t + EPV) : t + EPV == L)) {
             T* fs = static_cast<T*>(p.final_states_out) + b * p.final_states_stride[0] +
                     c * p.final_states_stride[1];
 #pragma unroll
-            for (int i = 0; i < H; ++i) {  // position L - H + i is window slot Lv + i - t
-                const float fv = RAG ? pick<H + EPV>(win, Lv + i - t) : win[EPV + i];  // aligned: t + EPV == L
-                st(fs, i * p.final_states_stride[2], (L - H + i >= 0) ? fv : 0.0f);
+            for (int i = 0; i < H; ++i) {  // position L - H + i is window slot L + i - t
+                const float fv = MODE != kRowsAligned ? pick<H + EPV>(win, L + i - t) : win[EPV + i];  // t + EPV == L
+                st(fs, i * p.final_states_stride[2], (L - H + i >= m) ? fv : 0.0f);
             }
         }
     }
@@ -217,7 +237,7 @@ __device__ __forceinline__ void fwd_rows_segment(const cc1d_fwd_params& p, int l
 // Item = (row, segment) with row = b * dim + c; four wavefronts per block take
 // four consecutive items, i.e. adjacent segments of a row or adjacent rows.
 // All index arithmetic is 32-bit (the launcher checks the ranges).
-template <typename T, int W, int VPT, bool SILU, bool SEQ, bool RAG>
+template <typename T, int W, int VPT, bool SILU, bool SEQ, int MODE>
 __global__ void __launch_bounds__(256) fwd_rows_vec(const FwdArgs a) {
     constexpr int SEG = 64 * VPT * elems16<T>::value;
     const cc1d_fwd_params& p = a.p;
@@ -229,19 +249,38 @@ __global__ void __launch_bounds__(256) fwd_rows_vec(const FwdArgs a) {
     const int32_t t0 = (int32_t)((item - row * (uint32_t)a.nseg) * SEG);
     const uint32_t b = a.dim_div.div(row);
     const uint32_t c = row - b * (uint32_t)p.dim;
-    constexpr int EPV = elems16<T>::value;
-    // ragged rows: the row starts m elements past a 16-byte boundary
-    int32_t m = 0;
-    if constexpr (RAG) {
+    int32_t m = 0;  // the row starts m elements past a 16-byte boundary
+    if constexpr (MODE == kRowsAlike) {
         const T* xrow = static_cast<const T*>(p.x) + (int64_t)b * p.x_stride[0] + (int64_t)c * p.x_stride[1];
-        m = (int32_t)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(xrow) / sizeof(T)) & (EPV - 1));
+        m = (int32_t)uniform32((uint32_t)(reinterpret_cast<uintptr_t>(xrow) / sizeof(T)) & (elems16<T>::value - 1));
     }
-    const int32_t Lv = (int32_t)p.seqlen + m;
-    if (RAG && t0 >= Lv) return;  // the row ends before this segment
-    if ((t0 > 0 || m == 0) && t0 + SEG <= Lv)
-        fwd_rows_segment<T, W, VPT, SILU, SEQ, true, RAG>(p, lane, b, c, t0, m);
+    const int32_t Le = (int32_t)p.seqlen + m;
+    if (MODE == kRowsAlike && t0 >= Le) return;  // the row ends before this segment
+    if ((t0 > 0 || m == 0) && t0 + SEG <= Le)
+        fwd_rows_segment<T, W, VPT, SILU, SEQ, true, MODE>(p, lane, b, c, t0, m, true);
     else
-        fwd_rows_segment<T, W, VPT, SILU, SEQ, false, RAG>(p, lane, b, c, t0, m);
+        fwd_rows_segment<T, W, VPT, SILU, SEQ, false, MODE>(p, lane, b, c, t0, m, true);
+}
+
+// Rows of nseg <= 32 vectors: a wavefront takes 64 / nseg (rounded down)
+// consecutive rows, lane l vector l % nseg of row l / nseg. With a wavefront
+// per row instead, a row of 64 bf16 kept 8 of 64 lanes busy. The window
+// before a vector comes from the previous lane as in fwd_rows_vec, nothing
+// (or initial_states) before a row's first; weights and bias are per-lane
+// reads here (rows differ).
+template <typename T, int W, bool SILU, bool SEQ>
+__global__ void __launch_bounds__(256) fwd_rows_short(const FwdArgs a) {
+    const cc1d_fwd_params& p = a.p;
+    const uint32_t wl = threadIdx.x & 63;
+    const uint32_t nv = (uint32_t)a.nseg, per = (uint32_t)a.chunk;  // vectors per row, rows per wavefront
+    const uint32_t r = a.nseg_div.div(wl);
+    const uint32_t row0 = uniform32(blockIdx.x * 4u + (threadIdx.x >> 6)) * per;
+    if (row0 >= (uint32_t)a.n_items) return;
+    const bool on = r < per && row0 + r < (uint32_t)a.n_items;
+    const uint32_t row = on ? row0 + r : row0;
+    const uint32_t b = a.dim_div.div(row);
+    const uint32_t c = row - b * (uint32_t)p.dim;
+    fwd_rows_segment<T, W, 1, SILU, SEQ, false, kRowsShort>(p, (int)(wl - r * nv), b, c, 0, 0, on);
 }
 
 // Channel-last (unit channel stride), tiled: a lane owns CPL adjacent
@@ -475,24 +514,29 @@ bool rows_vec_ok(const cc1d_fwd_params& p) {
     return true;
 }
 
-// ragged rows (a seqlen that is not a multiple of the vector, or rows that do
-// not start on a 16-byte boundary): unit time stride, and out laid out like x
-// modulo the vector -- the same element strides modulo EPV and bases a
-// multiple of 16 bytes apart -- so every row of out starts as far past a
-// 16-byte boundary as its row of x; seq_idx with a unit time stride
+// rows of any length at any element boundary: unit time stride is all they
+// need (seq_idx too, as 16-byte vectors of 4 ids are read from it)
 template <typename T>
-bool rows_ragged_ok(const cc1d_fwd_params& p) {
+bool rows_any_ok(const cc1d_fwd_params& p) {
     constexpr int64_t EPV = elems16<T>::value;
     if (p.width - 1 > EPV) return false;
     if (p.x_stride[2] != 1 || p.out_stride[2] != 1) return false;
-    if ((p.out_stride[0] - p.x_stride[0]) % EPV != 0 || (p.out_stride[1] - p.x_stride[1]) % EPV != 0) return false;
-    if ((reinterpret_cast<intptr_t>(p.out) - reinterpret_cast<intptr_t>(p.x)) % 16 != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.out)) % sizeof(T)) return false;
     if (p.seq_idx != nullptr && (p.seq_idx_stride[1] != 1 || reinterpret_cast<uintptr_t>(p.seq_idx) % 4 != 0))
         return false;
     const int64_t lim = (int64_t)1 << 31;
     if (p.seqlen + 64 * 4 * EPV + EPV >= lim) return false;
-    if (p.batch * p.dim * ceil_div(p.seqlen + EPV, 64 * EPV) * 4 >= ((int64_t)1 << 32)) return false;
+    if (p.batch * p.dim * ceil_div(p.seqlen + EPV, 64 * EPV) * 4 >= lim * 2) return false;
     return true;
+}
+
+// rows_any_ok, and out laid out like x modulo the vector: the same element
+// strides modulo EPV and bases a multiple of 16 bytes apart
+template <typename T>
+bool rows_alike(const cc1d_fwd_params& p) {
+    constexpr int64_t EPV = elems16<T>::value;
+    return (p.out_stride[0] - p.x_stride[0]) % EPV == 0 && (p.out_stride[1] - p.x_stride[1]) % EPV == 0 &&
+           (reinterpret_cast<intptr_t>(p.out) - reinterpret_cast<intptr_t>(p.x)) % 16 == 0;
 }
 
 // channel-last tiles: unit channel stride, CPL | dim, rows aligned to the
@@ -526,48 +570,82 @@ int launch_fwd(const cc1d_fwd_params& p, hipStream_t stream) {
                 a.p = p;
                 a.chunk = 0;
                 a.ngroups = 0;
-                a.ragged = 0;
                 const int64_t rows = p.batch * p.dim;
                 if constexpr (W - 1 <= EPV) {
                     const bool aligned = rows_vec_ok<T>(p);
-                    if (aligned || rows_ragged_ok<T>(p)) {
-                        a.ragged = aligned ? 0 : 1;
-                        // vectors a row spans: a ragged row may start up to EPV - 1
-                        // elements past a vector boundary
-                        const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
-                        const int64_t per = ceil_div(nvec, 64);
-                        int vpt = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
-                        // ragged rows (measured at C2's batch and dim; aligned ones
-                        // were faster without either): one segment of 4 vectors per
-                        // lane instead of two of 2 with the same lane slots when the
-                        // grid keeps 2048 wavefronts (L = 1031: 22.3 instead of
-                        // 25.1 us), and 2 instead of 4 when a row a
-                        // little longer than a multiple of the 4-vector segment would
-                        // leave its last one mostly empty and 2 take at most 85 % of
-                        // the lane slots (L = 2047: 34.2 instead of 37.6 us)
-                        if (!aligned && per == 3 && rows >= 2048) vpt = 4;
-                        else if (!aligned && vpt == 4 &&
-                                 ceil_div(nvec, (int64_t)128) * 128 * 100 <= ceil_div(nvec, (int64_t)256) * 256 * 85)
-                            vpt = 2;
-                        // a grid of fewer than 2048 wavefronts (2 per SIMD): half the
-                        // vectors per lane, twice the wavefronts (B = 1, D = 768,
-                        // L = 2048: 3.03 instead of 3.41 us; D = 512, L = 1024:
-                        // 2.40 instead of 2.53)
-                        if (vpt == 4 && rows * ceil_div(nvec, (int64_t)256) < 2048) vpt = 2;
-                        if (vpt == 2 && rows * ceil_div(nvec, (int64_t)128) < 2048) vpt = 1;
-                        a.nseg = ceil_div(nvec, 64 * (int64_t)vpt);
+                    if (aligned || rows_any_ok<T>(p)) {
+                        a.dim_div = FastDiv((uint32_t)p.dim);
+                        const int64_t least = ceil_div(p.seqlen, EPV);  // vectors from the row's first element on
+                        if (least <= kShortVecs && rows_any_ok<T>(p)) {
+                            a.nseg = least;
+                            a.chunk = 64 / least;
+                            a.n_items = rows;
+                            a.nseg_div = FastDiv((uint32_t)least);
+                            const dim3 grid((unsigned)ceil_div(ceil_div(rows, a.chunk), 4));
+                            return with_flag(p.seq_idx != nullptr, [&](auto qc) {
+                                return launch(fwd_rows_short<T, W, SILU, decltype(qc)::value>, grid, dim3(256), stream, a);
+                            });
+                        }
+                        // vectors per lane of rows of nvec vectors
+                        auto lanes = [&](int64_t nvec) {
+                            const int64_t per = ceil_div(nvec, 64);
+                            int vpt = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
+                            // rows off the 16-byte grid (measured at C2's batch and dim; aligned ones
+                            // were faster without either): one segment of 4 vectors per
+                            // lane instead of two of 2 with the same lane slots when the
+                            // grid keeps 2048 wavefronts (L = 1031: 22.3 instead of
+                            // 25.1 us), and 2 instead of 4 when a row a
+                            // little longer than a multiple of the 4-vector segment would
+                            // leave its last one mostly empty and 2 take at most 85 % of
+                            // the lane slots (L = 2049: 34.2 instead of 37.6 us)
+                            if (!aligned && per == 3 && rows >= 2048) vpt = 4;
+                            else if (!aligned && vpt == 4 &&
+                                     ceil_div(nvec, (int64_t)128) * 128 * 100 <= ceil_div(nvec, (int64_t)256) * 256 * 85)
+                                vpt = 2;
+                            // a grid of fewer than 2048 wavefronts (2 per SIMD): half the
+                            // vectors per lane, twice the wavefronts (B = 1, D = 768,
+                            // L = 2048: 3.03 instead of 3.41 us; D = 512, L = 1024:
+                            // 2.40 instead of 2.53)
+                            if (vpt == 4 && rows * ceil_div(nvec, (int64_t)256) < 2048) vpt = 2;
+                            if (vpt == 2 && rows * ceil_div(nvec, (int64_t)128) < 2048) vpt = 1;
+                            return vpt;
+                        };
+                        int vpt = lanes(least);
+                        a.nseg = ceil_div(least, 64 * (int64_t)vpt);
+                        bool alike = false;
+                        if (!aligned && rows_alike<T>(p)) {
+                            // a row that starts past a vector boundary may span one more
+                            const int64_t nvec = ceil_div(p.seqlen + EPV - 1, EPV);
+                            const int va = lanes(nvec);
+                            const int64_t na = ceil_div(nvec, 64 * (int64_t)va);
+                            // aligned vectors, unless that one more costs much of the lane
+                            // slots (16-bit types, us at C2's batch and dim, aligned ->
+                            // unaligned: L = 1023 21.9 -> 18.2, with seq_idx 35.8 -> 22.4, 511
+                            // 14.9 -> 13.1; ten times the batch 177 -> 152, 106 -> 102). A third
+                            // of them (L = 2047) pays only with seq_idx (50.1 -> 38.9): large
+                            // calls lose as much to unaligned stores (batch 40: 316 -> 330; fp32
+                            // 586 -> 646)
+                            const int64_t most = p.seq_idx != nullptr ? 85 : 60;  // % of the slots
+                            if (sizeof(T) == 4 || vpt * a.nseg * 100 > va * na * most) {
+                                alike = true;
+                                vpt = va;
+                                a.nseg = na;
+                            }
+                        }
                         a.n_items = rows * a.nseg;
                         a.nseg_div = FastDiv((uint32_t)a.nseg);
-                        a.dim_div = FastDiv((uint32_t)p.dim);
                         const dim3 grid((unsigned)ceil_div(a.n_items, 4));
                         return with_flag(p.seq_idx != nullptr, [&](auto qc) {
                             constexpr bool SEQ = decltype(qc)::value;
-                            return with_flag(a.ragged != 0, [&](auto rc) {
-                                constexpr bool RAG = decltype(rc)::value;
-                                if (vpt == 4) return launch(fwd_rows_vec<T, W, 4, SILU, SEQ, RAG>, grid, dim3(256), stream, a);
-                                if (vpt == 2) return launch(fwd_rows_vec<T, W, 2, SILU, SEQ, RAG>, grid, dim3(256), stream, a);
-                                return launch(fwd_rows_vec<T, W, 1, SILU, SEQ, RAG>, grid, dim3(256), stream, a);
-                            });
+                            auto go = [&](auto mc) {
+                                constexpr int MODE = decltype(mc)::value;
+                                if (vpt == 4) return launch(fwd_rows_vec<T, W, 4, SILU, SEQ, MODE>, grid, dim3(256), stream, a);
+                                if (vpt == 2) return launch(fwd_rows_vec<T, W, 2, SILU, SEQ, MODE>, grid, dim3(256), stream, a);
+                                return launch(fwd_rows_vec<T, W, 1, SILU, SEQ, MODE>, grid, dim3(256), stream, a);
+                            };
+                            if (aligned) return go(std::integral_constant<int, kRowsAligned>{});
+                            if (alike) return go(std::integral_constant<int, kRowsAlike>{});
+                            return go(std::integral_constant<int, kRowsAny>{});
                         });
                     }
                 }
