@@ -26,6 +26,9 @@
 //                     16-byte chunks: two adjacent lanes per (b, c) read the
 //                     two chunks that hold its window (one 32-byte access),
 //                     swap them, and write back the ones the window touches.
+//   update_ring    -- circular mode on lines of whole, aligned 64-byte granules:
+//                     four adjacent lanes per (b, c) read and write back the
+//                     granule (or two) that its window lies in.
 //   update_circ    -- other circular cases with up to 8 new tokens; one thread
 //                     per (b, c) with all loads issued before any store.
 //   update_generic -- everything else; one thread per (b, c).
@@ -640,6 +643,142 @@ __global__ void __launch_bounds__(256) update_circ_vec(const UpdArgs a) {
     }
 }
 
+// Circular mode on state lines of whole, 64-byte aligned granules (GE = 4 *
+// EPV elements): the window of W-1 history and Ls <= 8 new positions lies in
+// at most two granules. cache_seqlens is one value per batch entry, so where
+// the window starts and which granules it touches is wave-uniform (a
+// wavefront works on one entry). Four adjacent lanes read a channel's
+// granule, 16 bytes each, and put it into LDS, where any element can be
+// addressed: lane q of the four adds tokens q and q + 4 at their places and
+// computes their outputs from the window before them, then the granules that
+// received a token are read back and stored whole.
+//
+// What bounds it: memory, at the granularity of 128 bytes for reads (whatever
+// part of a line is asked for) and 64 for writes. Writing back only the
+// 16-byte chunks that change moves fewer bytes but costs more: with no
+// arithmetic, 256 x 5120 lines of 128 bytes take 62 us with one chunk of each
+// read and written (74 non-temporal), 49.7 with one granule (non-temporal;
+// 61 cached), 52.7 with the whole line. This kernel: C4b 53.8 us, 66.5 with
+// update_circ_vec. (Element places picked in registers instead of LDS, with
+// ds_bpermute and selects by wave-uniform indices, became 119 branches: 73 us.)
+template <typename T, int W, bool SILU, int NV>
+__global__ void __launch_bounds__(256) update_ring(const UpdArgs a) {
+    constexpr int H = W - 1;
+    constexpr int EPV = elems16<T>::value;
+    constexpr int GE = 4 * EPV;
+    constexpr int ES = (int)sizeof(T);
+    // a channel's granule takes 80 bytes of LDS: with 64 all 16 channels of a
+    // wavefront would meet in the same banks
+    constexpr int CHB = 80, GRB = 16 * CHB;  // bytes per channel, per 16 channels
+    __shared__ u32x4 lds[4][NV][2 * GRB / 16];
+    const cc1d_update_params& p = a.p;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3, ch = lane >> 2;
+    const uint32_t b = blockIdx.y, D = (uint32_t)p.dim;
+    const uint32_t cw = uniform32((blockIdx.x * 4u + wave) * (16u * NV));  // first channel
+    if (cw >= D) return;
+    const int Ls = (int)p.seqlen;
+    const int32_t S = (int32_t)p.state_len;
+    int64_t row = b;
+    if (p.conv_state_indices != nullptr) {
+        row = ld_uniform(p.conv_state_indices + b);
+        if (row >= p.state_rows) row = -1;  // out of the pool: as padding
+    }
+    int32_t cs = ld_uniform(p.cache_seqlens + b);
+    if ((uint32_t)cs >= (uint32_t)S) {  // floored modulo (torch.remainder)
+        cs = (int32_t)uniform32((uint32_t)(cs % S));
+        if (cs < 0) cs += S;
+    }
+    int32_t p0 = cs - H;  // first window position
+    if (p0 < 0) p0 += S;
+    const int32_t ng = S / GE, k0 = p0 / GE, k1 = k0 + 1 < ng ? k0 + 1 : 0;
+    const int O = p0 % GE;
+    const bool one = ng == 1;                     // the line is one granule: the window wraps inside it
+    const bool two = !one && O + H + Ls > GE;     // the window reaches into the granule after (its last token does)
+    const bool first = one || O + H < GE;         // new tokens start in the first one
+
+    uint32_t c[NV];
+    bool on[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const uint32_t ci = cw + 16 * i + ch;
+        on[i] = ci < D;
+        c[i] = on[i] ? ci : D - 1;  // lanes past the end read the last channel and store nothing
+    }
+    if (row < 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            T* __restrict__ orow = static_cast<T*>(p.out) + b * p.out_stride[0] + c[i] * p.out_stride[1];
+            for (int t = q; t < Ls; t += 4)
+                if (on[i]) st(orow, t * p.out_stride[2], 0.0f);
+        }
+        return;
+    }
+    T* __restrict__ sl = static_cast<T*>(p.conv_state) + row * p.conv_state_stride[0] + q * EPV;
+    u32x4 va[NV], vb[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) va[i] = vload_nt(sl + c[i] * p.conv_state_stride[1] + k0 * GE);
+    if (two) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < NV; ++i) vb[i] = vload_nt(sl + c[i] * p.conv_state_stride[1] + k1 * GE);
+    }
+    // lane q's tokens q and q + 4 (clamped into the burst), weights and bias, raw
+    T xt[NV][2], wr[NV][W], br[NV];
+    const int t0 = q < Ls ? q : Ls - 1, t1 = q + 4 < Ls ? q + 4 : Ls - 1;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const T* __restrict__ xr = static_cast<const T*>(p.x) + b * p.x_stride[0] + c[i] * p.x_stride[1];
+        xt[i][0] = xr[t0 * p.x_stride[2]];
+        xt[i][1] = xr[t1 * p.x_stride[2]];
+        const T* __restrict__ wp = static_cast<const T*>(p.weight) + (int64_t)c[i] * p.weight_stride[0];
+#pragma unroll
+        for (int k = 0; k < W; ++k) wr[i][k] = wp[k * p.weight_stride[1]];
+        br[i] = *(p.bias ? static_cast<const T*>(p.bias) + (int64_t)c[i] * p.bias_stride : wp);
+    }
+    // LDS byte of window element e of the lane's channel
+    const int wrap = one ? -GE * ES : GRB - GE * ES;
+    auto at = [&](int i, int e) -> T* {
+        const int off = ch * CHB + e * ES + (e >= GE ? wrap : 0);
+        return reinterpret_cast<T*>(reinterpret_cast<char*>(&lds[wave][i][0]) + off);
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        char* g = reinterpret_cast<char*>(&lds[wave][i][0]) + ch * CHB + q * 16;
+        *reinterpret_cast<u32x4*>(g) = va[i];
+        if (two) *reinterpret_cast<u32x4*>(g + GRB) = vb[i];
+    }
+    __builtin_amdgcn_wave_barrier();
+    // (the W-1 + Ls window positions are distinct: ring_ok keeps them within S)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        if (q < Ls) *at(i, O + H + q) = xt[i][0];
+        if (q + 4 < Ls) *at(i, O + H + q + 4) = xt[i][1];
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        float w[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k) w[k] = to_f32(wr[i][k]);
+        const float bias = p.bias ? to_f32(br[i]) : 0.0f;
+        T* __restrict__ orow = static_cast<T*>(p.out) + b * p.out_stride[0] + c[i] * p.out_stride[1];
+#pragma unroll
+        for (int r = 0; r < 8; r += 4) {
+            if (r >= Ls) break;  // wave-uniform; lane q: token r + q
+            const int t = r + q;
+            float win[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) win[k] = to_f32(*at(i, O + t + k));
+            float acc = conv_taps<W>(bias, w, win);
+            if constexpr (SILU) acc = silu(acc);
+            if (on[i] && t < Ls) st(orow, t * p.out_stride[2], acc);
+        }
+        const char* g = reinterpret_cast<const char*>(&lds[wave][i][0]) + ch * CHB + q * 16;
+        if (first && on[i]) vstore_nt(sl + c[i] * p.conv_state_stride[1] + k0 * GE, *reinterpret_cast<const u32x4*>(g));
+        if (two && on[i])
+            vstore_nt(sl + c[i] * p.conv_state_stride[1] + k1 * GE, *reinterpret_cast<const u32x4*>(g + GRB));
+    }
+}
+
 namespace {
 
 // update_lin: 16-byte vectors per lane (each wavefront covers 16 * EPV * kLinNV
@@ -661,6 +800,8 @@ constexpr int kDirNS = 1;
 // 4 entries x 4 wavefronts 7.08. The scattered-row copy does not gain from
 // wider workgroups (6.50 us with 1, 6.53 with 2, 4 or 5 wavefronts).
 constexpr int kDirWPG = 4;
+// update_ring: channels per quad of lanes
+constexpr int kRingNV = 2;
 
 template <typename T>
 bool lin_ok(const cc1d_update_params& p) {
@@ -697,6 +838,20 @@ bool circ_vec_ok(const cc1d_update_params& p) {
     if (!aligned16(p.conv_state)) return false;
     if (2 * p.batch * p.dim >= ((int64_t)1 << 31) || p.state_len >= ((int64_t)1 << 31)) return false;
     return true;
+}
+
+// granules: contiguous state lines of whole 64-byte aligned granules, up to 8
+// new tokens (W-1 + 8 elements reach into two granules at most)
+template <typename T>
+bool ring_ok(const cc1d_update_params& p) {
+    constexpr int64_t GE = 64 / (int64_t)sizeof(T);
+    if (p.cache_seqlens == nullptr || p.seqlen < 1 || p.seqlen > 8) return false;
+    if (p.width - 1 + p.seqlen > GE) return false;
+    if (p.state_len % GE != 0 || p.state_len >= ((int64_t)1 << 31)) return false;
+    if (p.conv_state_stride[2] != 1 || p.conv_state_stride[1] % GE || p.conv_state_stride[0] % GE) return false;
+    if (reinterpret_cast<uintptr_t>(p.conv_state) & 63u) return false;
+    // a grid of (channel groups, batch entries), 32-bit channels
+    return p.batch <= 65535 && p.dim < ((int64_t)1 << 31);
 }
 
 // tokens of x and out contiguous, a whole number of dwords, dword-aligned rows
@@ -757,8 +912,21 @@ int launch_update(const cc1d_update_params& p, hipStream_t stream) {
                 }
                 a.n_items = p.batch * p.dim;
                 const dim3 grid((unsigned)ceil_div(a.n_items, 256));
+                bool chunks = false;
+                if constexpr (W - 1 <= EPV) chunks = circ_vec_ok<T>(p);
+                // whole granules where the lines touched (128 bytes are read of each)
+                // do not stay in the 256 MB Infinity Cache from call to call, and
+                // wherever chunks cannot be used; below, chunks write a quarter of
+                // the bytes (bf16, S = 64, one token, us, chunks / granules: 256 x
+                // 5120 64.1 / 51.4, 256 x 2560 with three pools in turn 22.0 / 26.6)
+                const int64_t line = p.state_len * (int64_t)sizeof(T);
+                const int64_t touched = p.batch * p.dim * (line < 128 ? line : 128);
+                if (ring_ok<T>(p) && (!chunks || touched >= ((int64_t)96 << 20))) {
+                    const dim3 gr((unsigned)ceil_div(p.dim, 64 * kRingNV), (unsigned)p.batch);
+                    return launch(update_ring<T, W, SILU, kRingNV>, gr, dim3(256), stream, a);
+                }
                 if constexpr (W - 1 <= EPV) {
-                    if (circ_vec_ok<T>(p)) {
+                    if (chunks) {
                         a.n_items = 2 * p.batch * p.dim;  // two lanes per (b, c)
                         return with_flag(circ_dwords_ok<T>(p), [&](auto dc) {
                             return launch(update_circ_vec<T, W, SILU, decltype(dc)::value>,
