@@ -21,6 +21,9 @@ Differences in *where* work happens (results are the same):
   reference, and the same inputs give the same bits on every run.
 * ``dout`` keeps its layout when it already matches ``x`` (the kernels read
   any strides); only a mismatching layout is copied once.
+* an ordinary call -- plain GPU tensors, nothing tracing or transforming --
+  is checked, allocated, recorded for autograd and launched in native code
+  (``_host``); the ops and the autograd Function below serve every other one.
 * widths 6..9 with autograd are accepted at any seqlen (the reference needs
   seqlen % 1024 == 0 there, ``_fn.py:415-423``).
 """
@@ -29,6 +32,7 @@ from __future__ import annotations
 
 import torch
 
+from causal_conv1d_amd import _host
 from causal_conv1d_amd._dtype import _DTYPE_CODE
 from causal_conv1d_amd._native import native_bwd, native_bwd_typed, native_fwd
 
@@ -236,6 +240,12 @@ def causal_conv1d_fn(
 
     out: (batch, dim, seqlen)
     """
+    if getattr(x, "is_cuda", False) and not torch.compiler.is_compiling():
+        r = _host.native().fn(
+            x, weight, bias, seq_idx, initial_states, return_final_states, final_states_out, activation
+        )
+        if r is not NotImplemented:
+            return r
     if activation not in (None, "silu", "swish"):
         raise NotImplementedError("only activation in {None, 'silu', 'swish'} is supported")
     if x.dtype not in _DTYPE_CODE:

@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import torch
 
+from causal_conv1d_amd import _host
 from causal_conv1d_amd._dtype import _DTYPE_CODE
 from causal_conv1d_amd._native import native_update
 
@@ -39,6 +40,11 @@ def causal_conv1d_update(
 
     Returns: out, same shape as x.
     """
+    if getattr(x, "is_cuda", False) and not torch.compiler.is_compiling():
+        # an ordinary call, checked and launched in native code
+        out = _host.native().update(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices)
+        if out is not NotImplemented:
+            return out
     if activation not in (None, "silu", "swish"):
         raise NotImplementedError("only activation in {None, 'silu', 'swish'} is supported")
     if x.dtype not in _DTYPE_CODE:

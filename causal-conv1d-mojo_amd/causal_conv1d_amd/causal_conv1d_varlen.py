@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import torch
 
+from causal_conv1d_amd import _host
 from causal_conv1d_amd._native import native_varlen_states
 
 
@@ -26,6 +27,11 @@ def causal_conv1d_varlen_states(x: torch.Tensor, cu_seqlens: torch.Tensor, state
     Returns states: (batch, dim, state_len), dtype/device of x, allocated as
     (batch, state_len, dim) and transposed (unit stride along dim).
     """
+    if getattr(x, "is_cuda", False) and not torch.compiler.is_compiling():
+        # an ordinary call, checked and launched in native code
+        states = _host.native().varlen_states(x, cu_seqlens, state_len)
+        if states is not NotImplemented:
+            return states
     if x.dim() != 2:
         raise ValueError(f"x shape {tuple(x.shape)}: expected (total_tokens, dim)")
     if cu_seqlens.dim() != 1 or cu_seqlens.shape[0] < 1:

@@ -6,7 +6,9 @@ with hipcc (in parallel), then linked into
 ``extern "C"`` entry points of ``include/cc1d.h``. ``bench/cc1d_floor.hip``
 (bandwidth floors that ``bench.py`` times beside the kernels; measurement
 code, not part of the package) is linked on its own into
-``libcc1d_floor.so`` beside ``bench.py`` at the repository root.
+``libcc1d_floor.so`` beside ``bench.py`` at the repository root. The native
+host path, ``host/cc1d_host.cpp``, is compiled for the host against the
+running interpreter's torch into ``causal_conv1d_amd/_lib/cc1d_host.so``.
 
 Usage: ``python causal-conv1d-mojo_amd/csrc/build.py [--jobs N] [--verbose]``.
 """
@@ -18,6 +20,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -31,6 +34,9 @@ LIB_PATH = LIB_DIR / "libcc1d_amd.so"
 # bandwidth floors for bench.py (measurement only: built beside bench.py, outside the package)
 FLOOR_SRC = CSRC / "bench" / "cc1d_floor.hip"
 FLOOR_PATH = REPO / "libcc1d_floor.so"
+# host path: a CPython extension over libtorch, no device code
+HOST_SRC = CSRC / "host" / "cc1d_host.cpp"
+HOST_PATH = LIB_DIR / "cc1d_host.so"
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
@@ -85,9 +91,31 @@ def _link(objs: list[Path], out: Path, verbose: bool) -> None:
     os.replace(tmp, out)
 
 
+def _build_host(verbose: bool) -> None:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(HIPCC).resolve().parent.parent
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+        f"-I{INCLUDE}", "-isystem", str(root / "include"), "-isystem",
+        str(root / "include" / "torch" / "csrc" / "api" / "include"), "-isystem", str(rocm / "include"),
+        "-isystem", sysconfig.get_paths()["include"], str(HOST_SRC), "-o", str(tmp),
+        f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+    ]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"the host path did not compile:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     """Compile every HIP source and link the shared library (and the bench's
-    floor library). Returns the product library's path."""
+    floor library), and compile the host path. Returns the product library's path."""
     if HIPCC is None or not Path(HIPCC).exists():
         raise RuntimeError("hipcc not found; set HIPCC or install ROCm")
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
@@ -95,7 +123,9 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     srcs = _sources() + [FLOOR_SRC]
     jobs = jobs or min(len(srcs), max(1, os.cpu_count() or 1))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
+        host.result()
     _link(objs[:-1], LIB_PATH, verbose)
     _link(objs[-1:], FLOOR_PATH, verbose)
     return LIB_PATH
