@@ -971,7 +971,7 @@ template <typename T, int W, int CPL> struct ClWeights {
 // c0 - H + i (clamped into [0, L)), read through the scalar cache (NI = G + H
 // with seq_idx, else 1 unused).
 template <typename T, int CPL, int G, int NI> struct ClChunk {
-    Lanes<T, CPL> x[G], g[G];
+    Lanes<T> x[G], g[G];
     int32_t ids[NI];
 };
 
@@ -1002,15 +1002,13 @@ template <int W, int CPL> struct ClWalk {
 // Non-temporal: a walk reads each row once (the few rows a neighbouring run
 // reads again are its H-row prime and tail); at C3 the backward took 37.3 /
 // 38.5 us with non-temporal row loads against 40.5 / 41.3 us with cached ones.
-template <typename T, int CPL> __device__ __forceinline__ Lanes<T, CPL> row_load(const T* base, uint32_t off) {
-    static_assert(Lanes<T, CPL>::ND == 1, "one dword per lane");
-    Lanes<T, CPL> v;
-    v.d[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(base) + off));
+template <typename T> __device__ __forceinline__ Lanes<T> row_load(const T* base, uint32_t off) {
+    Lanes<T> v;
+    v.template load<true>(reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off));
     return v;
 }
-template <typename T, int CPL> __device__ __forceinline__ void row_store_nt(T* base, uint32_t off, const Lanes<T, CPL>& v) {
-    static_assert(Lanes<T, CPL>::ND == 1, "one dword per lane");
-    __builtin_nontemporal_store(v.d[0], reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(base) + off));
+template <typename T> __device__ __forceinline__ void row_store_nt(T* base, uint32_t off, const Lanes<T>& v) {
+    v.template store<true>(reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off));
 }
 
 // Kernel: the WPB wavefronts of a block take WPB consecutive runs of the same
@@ -1041,8 +1039,14 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
     const int32_t L = (int32_t)p.seqlen;
     const int32_t t0 = (int32_t)uniform32((tg * WPB + wave) * R);
     const int32_t cw0 = (int32_t)(grp * NC);
-    const int32_t c0 = cw0 + lane * CPL;
-    const bool active = c0 < (int32_t)p.dim;
+    const bool active = cw0 + lane * CPL < (int32_t)p.dim;
+    // the last lane of an odd number of 16-bit channels takes the last CPL ones
+    // (`shifted`): the channel it shares with the lane before gets the same dx
+    // from both, and its share of the sums is dropped below. cb: the channel
+    // the wavefront's row addresses start from
+    const int32_t cb = cw0 + CPL <= (int32_t)p.dim ? cw0 : (int32_t)p.dim - CPL;
+    const bool shifted = active && cw0 + lane * CPL + CPL > (int32_t)p.dim;
+    const int32_t c0 = shifted ? (int32_t)p.dim - CPL : cw0 + lane * CPL;
 
     ClWalk<W, CPL> s;
 #pragma unroll
@@ -1054,13 +1058,13 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
     if (t0 < L) {  // runs past the end only join the block reduction
         const int32_t xs2 = (int32_t)p.x_stride[2], gs2 = (int32_t)p.dout_stride[2];
         const int32_t ds2 = (int32_t)p.dx_stride[2];
-        // lanes past the last channel read channel 0 of the group's rows (in
+        // lanes past the last channel read the group's first ones (in
         // bounds); they store nothing and their partials are dropped
-        const int32_t lo = active ? lane * CPL : 0;
+        const int32_t lo = active ? c0 - cb : 0;
         const uint32_t lob = (uint32_t)lo * (uint32_t)sizeof(T);  // the lane's byte offset in a row
-        const T* __restrict__ xb = static_cast<const T*>(p.x) + b * p.x_stride[0] + cw0;
-        const T* __restrict__ gb = static_cast<const T*>(p.dout) + b * p.dout_stride[0] + cw0;
-        T* __restrict__ dxb = static_cast<T*>(p.dx) + b * p.dx_stride[0] + cw0;
+        const T* __restrict__ xb = static_cast<const T*>(p.x) + b * p.x_stride[0] + cb;
+        const T* __restrict__ gb = static_cast<const T*>(p.dout) + b * p.dout_stride[0] + cb;
+        T* __restrict__ dxb = static_cast<T*>(p.dx) + b * p.dx_stride[0] + cb;
         const int32_t* __restrict__ sr = SEQ ? p.seq_idx + b * p.seq_idx_stride[0] : nullptr;
         const int32_t ss1 = SEQ ? (int32_t)p.seq_idx_stride[1] : 0;
         auto clampL = [&](int32_t t) { return t < 0 ? 0 : (t < L ? t : L - 1); };
@@ -1071,8 +1075,8 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
                 const int32_t t = clampL(cs + j);
-                ch.x[j] = row_load<T, CPL>(xb, (uint32_t)(t * xs2) * (uint32_t)sizeof(T) + lob);
-                ch.g[j] = row_load<T, CPL>(gb, (uint32_t)(t * gs2) * (uint32_t)sizeof(T) + lob);
+                ch.x[j] = row_load<T>(xb, (uint32_t)(t * xs2) * (uint32_t)sizeof(T) + lob);
+                ch.g[j] = row_load<T>(gb, (uint32_t)(t * gs2) * (uint32_t)sizeof(T) + lob);
             }
             if constexpr (SEQ) {
                 constexpr int NI = G + H;
@@ -1090,12 +1094,12 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
         };
 
         // x rows t0-H .. t0-1 (zero before the sequence, or initial_states)
-        Lanes<T, CPL> prime[H];
+        Lanes<T> prime[H];
         const bool prime_rows = t0 >= H;
         if (prime_rows) {
 #pragma unroll
             for (int k = 0; k < H; ++k)
-                prime[k] = row_load<T, CPL>(xb, (uint32_t)((t0 - H + k) * xs2) * (uint32_t)sizeof(T) + lob);
+                prime[k] = row_load<T>(xb, (uint32_t)((t0 - H + k) * xs2) * (uint32_t)sizeof(T) + lob);
         }
         ClWeights<T, W, CPL> wt;
         wt.load(p, c0, active);
@@ -1150,9 +1154,9 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
             }
         };
         auto store_dx = [&](int32_t pos, const float* o) {
-            Lanes<T, CPL> ov;
+            Lanes<T> ov;
             ov.set(o);
-            row_store_nt<T, CPL>(dxb, (uint32_t)(pos * ds2) * (uint32_t)sizeof(T) + lob, ov);
+            row_store_nt<T>(dxb, (uint32_t)(pos * ds2) * (uint32_t)sizeof(T) + lob, ov);
         };
 
         // NS steps of chunk ch at cs, ungated (the chunk's window [cs-H, cs+NS+H)
@@ -1166,7 +1170,7 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
 #pragma unroll
             for (int j = 0; j < NS; ++j) {
                 float xc[CPL], dn[CPL], o[CPL];
-                const Lanes<T, CPL> xl = ch.x[j], gl = ch.g[j];
+                const Lanes<T> xl = ch.x[j], gl = ch.g[j];
 #pragma unroll
                 for (int e = 0; e < CPL; ++e) {
                     xc[e] = xl.get(e);
@@ -1219,7 +1223,7 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
                 }
                 const bool dead = !in || idp < 0;
                 float xc[CPL], dn[CPL];
-                const Lanes<T, CPL> xl = ch.x[j], gl = ch.g[j];
+                const Lanes<T> xl = ch.x[j], gl = ch.g[j];
 #pragma unroll
                 for (int e = 0; e < CPL; ++e) {
                     xc[e] = in ? xl.get(e) : 0.0f;
@@ -1350,6 +1354,17 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
                 for (int k = 0; k < W; ++k) s.pw[k][e] = 0.0f;
             }
         }
+        if constexpr (CPL == 2) {
+            if (shifted) {  // the last channel's sums go to its own place, the lane's first
+                s.pb[0] = s.pb[1];
+                s.pb[1] = 0.0f;
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    s.pw[k][0] = s.pw[k][1];
+                    s.pw[k][1] = 0.0f;
+                }
+            }
+        }
     }
 
     // ---- weight / bias gradient: sum the block's runs in LDS, then
@@ -1458,18 +1473,27 @@ bool rows_alike(const cc1d_bwd_params& p) {
     return (reinterpret_cast<intptr_t>(p.dout) - x) % 16 == 0 && (reinterpret_cast<intptr_t>(p.dx) - x) % 16 == 0;
 }
 
-// channel-last tiles: unit channel stride, CPL | dim, rows aligned to the
-// CPL-channel lane vector, 32-bit positions inside a batch
+// whole dwords of channels: CPL | dim, every row of x, dout and dx on a 4-byte boundary
 template <typename T, int CPL>
-bool cl_ok(const cc1d_bwd_params& p) {
+bool cl_dwords(const cc1d_bwd_params& p) {
     constexpr int64_t NB = CPL * (int64_t)sizeof(T);
-    if (p.x_stride[1] != 1 || p.dout_stride[1] != 1 || p.dx_stride[1] != 1) return false;
     if (p.dim % CPL != 0) return false;
     if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.dout) |
          reinterpret_cast<uintptr_t>(p.dx)) % NB)
         return false;
-    if (p.x_stride[0] % CPL || p.x_stride[2] % CPL || p.dout_stride[0] % CPL || p.dout_stride[2] % CPL ||
-        p.dx_stride[0] % CPL || p.dx_stride[2] % CPL)
+    return !(p.x_stride[0] % CPL || p.x_stride[2] % CPL || p.dout_stride[0] % CPL || p.dout_stride[2] % CPL ||
+             p.dx_stride[0] % CPL || p.dx_stride[2] % CPL);
+}
+
+// channel-last runs: unit channel stride, at least a lane's CPL channels,
+// 32-bit positions inside a batch
+template <typename T, int CPL>
+bool cl_ok(const cc1d_bwd_params& p) {
+    constexpr int64_t NB = CPL * (int64_t)sizeof(T);
+    if (p.x_stride[1] != 1 || p.dout_stride[1] != 1 || p.dx_stride[1] != 1) return false;
+    if (p.dim < CPL) return false;
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.dout) | reinterpret_cast<uintptr_t>(p.dx)) %
+        sizeof(T))
         return false;
     const int64_t span = p.seqlen + kClWPB * kClR + 16;  // past the furthest run start
     const int64_t lim = (int64_t)1 << 31;
@@ -1483,7 +1507,7 @@ bool cl_ok(const cc1d_bwd_params& p) {
         span * p.dx_stride[2] * (int64_t)sizeof(T) >= blim)
         return false;
     if (p.seq_idx != nullptr && span * p.seq_idx_stride[1] >= lim) return false;
-    if (p.batch * ceil_div(p.dim / CPL, 64) * ceil_div(p.seqlen, kClR * kClWPB) >= lim) return false;
+    if (p.batch * ceil_div(p.dim, (int64_t)(64 * CPL)) * ceil_div(p.seqlen, kClR * kClWPB) >= lim) return false;
     return true;
 }
 
@@ -1517,6 +1541,11 @@ inline int rows_vpt(int64_t nvec, int64_t rows) {
     int vpt = per >= 4 || (per == 3 && rows >= 2048) ? 4 : (per >= 2 ? 2 : 1);
     if (vpt == 4 && ceil_div(nvec, 128) * 128 * 100 <= ceil_div(nvec, 256) * 256 * 85) vpt = 2;
     return vpt;
+}
+
+// workspace of a call in the generic kernel's time chunks
+inline int64_t chunk_floats(const cc1d_bwd_params& p) {
+    return p.batch * p.dim * ceil_div(p.seqlen, (int64_t)kGenericChunk) * (p.width + 1);
 }
 
 template <typename T, int W>
@@ -1580,7 +1609,7 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
     if (cl_ok<T, CPL>(p)) {
         pl.kind = kBwdCl;
         pl.cpl = CPL;
-        pl.a.groups = ceil_div(p.dim / CPL, 64);
+        pl.a.groups = ceil_div(p.dim, (int64_t)(64 * CPL));
         // run length: a wavefront walks its run chunk by chunk, each chunk's
         // loads in flight behind the previous one's arithmetic, so a run takes
         // about the same time at any problem size (memory latency per chunk);
@@ -1600,7 +1629,13 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
         pl.blocks = p.batch * pl.a.groups * pl.a.nseg;
         pl.records = pl.blocks;
         pl.rec_floats = 64 * CPL * (W + 1);
-        return pl;
+        // rows off the dword grid: where the records fit into the workspace of
+        // the time chunks that such calls are sized by (reserved_floats; all but
+        // a few channels' ones do)
+        if (cl_dwords<T, CPL>(p) || pl.records * pl.rec_floats <= chunk_floats(p)) return pl;
+        pl.rec_floats = W + 1;
+        pl.a.groups = 0;
+        pl.cpl = 0;
     }
     pl.kind = kBwdGeneric;
     pl.a.chunk = kGenericChunk;
@@ -1612,24 +1647,26 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
 }
 
 // The workspace of a call: what cc1d_bwd_workspace_floats tells the caller and
-// cc1d_bwd_typed asks for. For rows it depends on sizes and layout alone and
-// not on the launch geometry -- segments of the vectors that a row spans, or
-// time chunks where the tensors lie unlike each other -- so that a size a
-// program has stored, or a problem that fits the static scratch, stays good
-// when a kernel splits rows another way. Every plan's records fit: kRowsShort
-// has one per row, kRowsAny at most one per 64 steps.
+// cc1d_bwd_typed asks for. It depends on sizes and layout alone and not on
+// which kernel a call takes -- segments of the vectors that a row spans, runs
+// of whole dwords of channels, else time chunks -- so that a size a program
+// has stored, or a problem that fits the static scratch, stays good when a
+// kernel takes more layouts or splits rows another way. Every plan's records
+// fit: kRowsShort has one per row, kRowsAny at most one per 64 steps, and
+// channels off the dword grid are only taken where they do.
 template <typename T, int W>
 int64_t reserved_floats(const cc1d_bwd_params& p, const BwdPlan& pl) {
-    if (pl.kind != kBwdRows || pl.mode == kRowsAligned || pl.mode == kRowsAlike) return pl.records * pl.rec_floats;
     constexpr int64_t EPV = elems16<T>::value;
-    const int64_t rows = p.batch * p.dim;
-    const bool aligned = rows_vec_ok<T>(p);
-    int64_t n = ceil_div(p.seqlen, (int64_t)kGenericChunk);
-    if (aligned || rows_alike<T>(p)) {
-        const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
-        n = ceil_div(nvec, 64 * (int64_t)rows_vpt(nvec, rows));
+    if (pl.kind == kBwdCl) {
+        constexpr int CPL = 4 / (int)sizeof(T);
+        return cl_dwords<T, CPL>(p) ? pl.records * pl.rec_floats : chunk_floats(p);
     }
-    return rows * n * pl.rec_floats;
+    if (pl.kind != kBwdRows || pl.mode == kRowsAligned || pl.mode == kRowsAlike) return pl.records * pl.rec_floats;
+    const bool aligned = rows_vec_ok<T>(p);
+    if (!aligned && !rows_alike<T>(p)) return chunk_floats(p);
+    const int64_t rows = p.batch * p.dim;
+    const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
+    return rows * ceil_div(nvec, 64 * (int64_t)rows_vpt(nvec, rows)) * pl.rec_floats;
 }
 
 template <typename T, int W, bool SILU>

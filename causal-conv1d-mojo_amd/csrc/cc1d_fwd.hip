@@ -296,7 +296,8 @@ template <typename T, int W, int CPL, int TS, bool SILU, bool SEQ>
 __global__ void __launch_bounds__(256) fwd_cl(const FwdArgs a) {
     constexpr int H = W - 1;
     constexpr int NR = TS + H;
-    using V = Lanes<T, CPL>;
+    using V = Lanes<T>;
+    static_assert(V::N == CPL, "a dword of channels per lane");
     const cc1d_fwd_params& p = a.p;
     const int lane = threadIdx.x & 63;
     const uint32_t item = uniform32(blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -307,8 +308,11 @@ __global__ void __launch_bounds__(256) fwd_cl(const FwdArgs a) {
     const uint32_t tile = rest % ntiles;
     const uint32_t b = rest / ntiles;
     const int32_t L = (int32_t)p.seqlen;
-    const int32_t c0 = (int32_t)((g * 64 + lane) * CPL);
-    const bool active = c0 < (int32_t)p.dim;
+    const int32_t cl = (int32_t)((g * 64 + lane) * CPL);
+    const bool active = cl < (int32_t)p.dim;
+    // the last lane of an odd number of 16-bit channels takes the last CPL ones:
+    // the channel it shares with the lane before is computed and stored twice, alike
+    const int32_t c0 = cl + CPL <= (int32_t)p.dim ? cl : (int32_t)p.dim - CPL;
     const int32_t t0 = (int32_t)(tile * TS);
     const int32_t xs2 = (int32_t)p.x_stride[2], os2 = (int32_t)p.out_stride[2];
     const T* __restrict__ xb = static_cast<const T*>(p.x) + b * p.x_stride[0] + c0;
@@ -539,20 +543,18 @@ bool rows_alike(const cc1d_fwd_params& p) {
            (reinterpret_cast<intptr_t>(p.out) - reinterpret_cast<intptr_t>(p.x)) % 16 == 0;
 }
 
-// channel-last tiles: unit channel stride, CPL | dim, rows aligned to the
-// CPL-channel lane vector, 32-bit positions inside a batch
+// channel-last tiles: unit channel stride, at least a lane's CPL channels,
+// 32-bit positions inside a batch
 template <typename T, int CPL>
 bool cl_ok(const cc1d_fwd_params& p) {
-    constexpr int64_t NB = CPL * (int64_t)sizeof(T);
     if (p.x_stride[1] != 1 || p.out_stride[1] != 1) return false;
-    if (p.dim % CPL != 0) return false;
-    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.out)) % NB) return false;
-    if (p.x_stride[0] % CPL || p.x_stride[2] % CPL || p.out_stride[0] % CPL || p.out_stride[2] % CPL) return false;
+    if (p.dim < CPL) return false;
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.out)) % sizeof(T)) return false;
     const int64_t span = p.seqlen + kClTS + 16;  // furthest row a tile touches
     const int64_t lim = (int64_t)1 << 31;
     if (p.dim >= lim || span * p.x_stride[2] >= lim || span * p.out_stride[2] >= lim) return false;
     if (p.seq_idx != nullptr && span * p.seq_idx_stride[1] >= lim) return false;
-    if (p.batch * ceil_div(p.dim / CPL, 64) * ceil_div(p.seqlen, kClTS) >= lim * 2) return false;
+    if (p.batch * ceil_div(p.dim, (int64_t)(64 * CPL)) * ceil_div(p.seqlen, kClTS) >= lim * 2) return false;
     return true;
 }
 
@@ -651,7 +653,7 @@ int launch_fwd(const cc1d_fwd_params& p, hipStream_t stream) {
                 }
                 constexpr int CPL = 4 / (int)sizeof(T);
                 if (cl_ok<T, CPL>(p)) {
-                    a.ngroups = ceil_div(p.dim / CPL, 64);
+                    a.ngroups = ceil_div(p.dim, (int64_t)(64 * CPL));
                     // 8-step tiles when 16-step ones would give fewer than 4096
                     // wavefronts: a tile is one round trip to memory, so a small
                     // grid gains from twice the wavefronts (bf16, B = 1, D = 768,
