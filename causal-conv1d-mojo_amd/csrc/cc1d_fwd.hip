@@ -318,6 +318,37 @@ __global__ void __launch_bounds__(256) fwd_cl(const FwdArgs a) {
     const T* __restrict__ xb = static_cast<const T*>(p.x) + b * p.x_stride[0] + c0;
     T* __restrict__ ob = static_cast<T*>(p.out) + b * p.out_stride[0] + c0;
 
+    // with seq_idx, and for fp32: ids, weights and bias go out before the rows
+    // (raw, so that no conversion waits for them here). Loads complete in
+    // order, so a row's outputs can then be computed as soon as that row has
+    // arrived (us, rows first -> last: bf16 1 x 4096 x 8192 with seq_idx 30.0 ->
+    // 26.8, 1536 x 2048 6.6 -> 5.6; fp32 4 x 2048 x 2000 27.0 -> 24.2). 16-bit
+    // types without seq_idx are quicker with the rows first below C3's size
+    // (4 x 2048 x 2000 15.8 against 16.3)
+    constexpr bool PARAMS_FIRST = SEQ || sizeof(T) == 4;
+    int32_t lid = 0;
+    if constexpr (SEQ) {
+        // lane i < NR reads the id of position t0 - H + i (clamped address,
+        // -1 outside the row); the window's ids then reach every lane through
+        // readlane, with no dependent scalar reads.
+        static_assert(NR <= 64, "the id window must fit in one wavefront");
+        const int32_t* sr = p.seq_idx + b * p.seq_idx_stride[0];
+        const int32_t s = t0 - H + lane;
+        lid = sr[(s < 0 ? 0 : (s < L ? s : L - 1)) * (int32_t)p.seq_idx_stride[1]];
+    }
+    T wr[W][CPL], br[CPL];
+    if constexpr (PARAMS_FIRST) {
+#pragma unroll
+        for (int e = 0; e < CPL; ++e) {
+            const int64_t c = active ? c0 + e : 0;
+            const T* wp = static_cast<const T*>(p.weight) + c * p.weight_stride[0];
+#pragma unroll
+            for (int k = 0; k < W; ++k) wr[k][e] = wp[k * p.weight_stride[1]];
+            br[e] = *(p.bias ? static_cast<const T*>(p.bias) + c * p.bias_stride : wp);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
     V xv[NR];
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
@@ -344,23 +375,23 @@ __global__ void __launch_bounds__(256) fwd_cl(const FwdArgs a) {
     float w[W][CPL], bias[CPL];
 #pragma unroll
     for (int e = 0; e < CPL; ++e) {
-        const int64_t c = active ? c0 + e : 0;
+        if constexpr (PARAMS_FIRST) {
 #pragma unroll
-        for (int k = 0; k < W; ++k)
-            w[k][e] = ld(static_cast<const T*>(p.weight), c * p.weight_stride[0] + k * p.weight_stride[1]);
-        bias[e] = p.bias ? ld(static_cast<const T*>(p.bias), c * p.bias_stride) : 0.0f;
+            for (int k = 0; k < W; ++k) w[k][e] = to_f32(wr[k][e]);
+            bias[e] = p.bias ? to_f32(br[e]) : 0.0f;
+        } else {
+            const int64_t c = active ? c0 + e : 0;
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+                w[k][e] = ld(static_cast<const T*>(p.weight), c * p.weight_stride[0] + k * p.weight_stride[1]);
+            bias[e] = p.bias ? ld(static_cast<const T*>(p.bias), c * p.bias_stride) : 0.0f;
+        }
     }
 
     int32_t id[NR];
     bool one_id = true;
     if constexpr (SEQ) {
-        // lane i < NR reads the id of position t0 - H + i (clamped address,
-        // -1 outside the row); the window's ids then reach every lane through
-        // readlane, with no dependent scalar reads.
-        static_assert(NR <= 64, "the id window must fit in one wavefront");
-        const int32_t* sr = p.seq_idx + b * p.seq_idx_stride[0];
         const int32_t s = t0 - H + lane;
-        int32_t lid = sr[(s < 0 ? 0 : (s < L ? s : L - 1)) * (int32_t)p.seq_idx_stride[1]];
         if (s < 0 || s >= L) lid = -1;
         const int32_t id_cur = __builtin_amdgcn_readlane(lid, H);
         // rows outside [0, L) hold zeros (seq_idx excludes initial_states) or
