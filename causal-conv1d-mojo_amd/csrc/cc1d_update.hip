@@ -11,12 +11,16 @@
 //   out-of-pool index zeroes out[b] and leaves the pool untouched.
 //
 // Kernels
-//   update_dir     -- linear mode, one token, S == W-1 <= 4, channel-contiguous
+//   update_dir     -- linear mode, one token, S == W-1 <= 4 or S == W, channel-contiguous
 //                     x / out and contiguous state rows: a lane owns one dword
 //                     of x (2 bf16/fp16 channels, 1 fp32) of two batch
-//                     entries and loads the channels' state span (H dwords)
+//                     entries and loads the channels' state span (S dwords)
 //                     directly, one load per span; no LDS; four wavefronts
 //                     (channel groups) per workgroup.
+//   update_step    -- linear mode, one token, state with unit channel stride (a
+//                     step's channels together, as causal_conv1d_varlen_states
+//                     returns it): a lane owns one dword of channels of every
+//                     step.
 //   update_lin     -- the same for W > 5: one token, S == W-1, channel-contiguous x /
 //                     out and contiguous state rows: one wavefront per (batch
 //                     entry, 16 * EPV channels) moves the group's state and x
@@ -280,22 +284,22 @@ __global__ void __launch_bounds__(64) update_lin(const LinArgs<T> a) {
     }
 }
 
-// Linear mode, seqlen 1, state_len == W-1 (H <= 4): a lane owns NS dwords of
+// Linear mode, seqlen 1, state_len S == W-1 (H <= 4) or W: a lane owns NS dwords of
 // x (CPL channels each: 2 bf16/fp16, 1 fp32; dwords lane, lane + 64, ...) and
-// reads their H-dword state spans directly, one dword-vector load per span;
+// reads their S-dword state spans directly, one dword-vector load per span;
 // consecutive lanes hold consecutive spans, so each load instruction covers
-// 64 * 4H contiguous bytes. No LDS and no shuffle between the loads, the
+// 64 * 4S contiguous bytes. No LDS and no shuffle between the loads, the
 // arithmetic and the stores. A wavefront takes 64 * NS * CPL channels of BPW
 // batch entries, a workgroup WPG consecutive channel groups of the same
 // entries (grid: workgroups along the channels x batch-entry groups); x first, then
 // the BPW pool indices (scalar loads) behind a scheduling fence, then the
 // state spans, then the weights and bias (cache-resident), all before any
 // arithmetic.
-template <typename T, int W, int BPW, int NS, int WPG, bool SILU, bool HAS_BIAS, bool HAS_IDX>
+template <typename T, int W, int S, int BPW, int NS, int WPG, bool SILU, bool HAS_BIAS, bool HAS_IDX>
 __global__ void __launch_bounds__(64 * WPG) update_dir(const LinArgs<T> a) {
     constexpr int H = W - 1;
     constexpr int CPL = 4 / (int)sizeof(T);
-    static_assert(H >= 1 && H <= 4, "one dword vector of state per span");
+    static_assert(H >= 1 && H <= 4 && (S == H || S == W), "a few dwords of state per span");
     const int lane = threadIdx.x & 63;
     const uint32_t grp = blockIdx.x * WPG + (threadIdx.x >> 6);  // channel group of this wavefront
     uint32_t c[NS];
@@ -343,15 +347,15 @@ __global__ void __launch_bounds__(64 * WPG) update_dir(const LinArgs<T> a) {
 #pragma unroll
         for (int q = 0; q < BPW; ++q) row[q] = (int32_t)min(b0 + q, nb - 1);
     }
-    uint32_t st[BPW][NS][H];
+    uint32_t st[BPW][NS][S];
 #pragma unroll
     for (int q = 0; q < BPW; ++q) {
         const T* srow = a.conv_state + (size_t)(row[q] >= 0 ? row[q] : 0) * a.state_row;
 #pragma unroll
         for (int u = 0; u < NS; ++u) {
-            const uint32_t* sp = reinterpret_cast<const uint32_t*>(srow + (size_t)c[u] * H);
+            const uint32_t* sp = reinterpret_cast<const uint32_t*>(srow + (size_t)c[u] * S);
 #pragma unroll
-            for (int i = 0; i < H; ++i) st[q][u][i] = __builtin_nontemporal_load(&sp[i]);
+            for (int i = 0; i < S; ++i) st[q][u][i] = __builtin_nontemporal_load(&sp[i]);
         }
     }
     // weights and bias (cache-resident) after the state loads: they arrive
@@ -377,16 +381,16 @@ __global__ void __launch_bounds__(64 * WPG) update_dir(const LinArgs<T> a) {
     for (int q = 0; q < BPW; ++q) {
 #pragma unroll
         for (int u = 0; u < NS; ++u) {
-            uint32_t sraw[CPL * H], nraw[CPL * H];
+            uint32_t sraw[CPL * S], nraw[CPL * S];
 #pragma unroll
-            for (int n = 0; n < CPL * H; ++n) sraw[n] = elem(st[q][u], n);
+            for (int n = 0; n < CPL * S; ++n) sraw[n] = elem(st[q][u], n);
             float o[CPL];
 #pragma unroll
             for (int e = 0; e < CPL; ++e) {
                 const uint32_t xb = elem(&xd[q][u], e);
                 float win[W], w[W];
 #pragma unroll
-                for (int i = 0; i < H; ++i) win[i] = as_f32(sraw[e * H + i]);
+                for (int i = 0; i < H; ++i) win[i] = as_f32(sraw[e * S + S - H + i]);
                 win[H] = as_f32(xb);
 #pragma unroll
                 for (int k = 0; k < W; ++k) w[k] = as_f32(elem(wd[u], e * W + k));
@@ -395,7 +399,7 @@ __global__ void __launch_bounds__(64 * WPG) update_dir(const LinArgs<T> a) {
                 if constexpr (SILU) acc = silu(acc);
                 o[e] = acc;
 #pragma unroll
-                for (int i = 0; i < H; ++i) nraw[e * H + i] = i + 1 < H ? sraw[e * H + i + 1] : xb;
+                for (int i = 0; i < S; ++i) nraw[e * S + i] = i + 1 < S ? sraw[e * S + i + 1] : xb;
             }
             uint32_t od;
             if constexpr (CPL == 1) od = __float_as_uint(o[0]);
@@ -405,13 +409,99 @@ __global__ void __launch_bounds__(64 * WPG) update_dir(const LinArgs<T> a) {
                 __builtin_nontemporal_store(od, reinterpret_cast<uint32_t*>(a.out + (size_t)(b0 + q) * a.out_row + c[u]));
                 if (row[q] >= 0) {
                     uint32_t* sp = reinterpret_cast<uint32_t*>(a.conv_state + (size_t)row[q] * a.state_row +
-                                                               (size_t)c[u] * H);
+                                                               (size_t)c[u] * S);
 #pragma unroll
-                    for (int i = 0; i < H; ++i)
+                    for (int i = 0; i < S; ++i)
                         __builtin_nontemporal_store(CPL == 1 ? nraw[i] : (nraw[2 * i] | (nraw[2 * i + 1] << 16)), &sp[i]);
                 }
             }
         }
+    }
+}
+
+// Arguments of update_step (see LinArgs).
+template <typename T> struct StepArgs {
+    LinArgs<T> l;
+    uint32_t state_step;  // stride (elements) of a state row's steps
+    int32_t S;            // steps of a state row
+};
+
+// Linear mode, seqlen 1, unit channel stride of x, out and the state: a lane
+// owns one dword of channels (CPL) of BPW batch entries and of each of their S
+// steps, so every access of a wavefront is 256 contiguous bytes. Load order as
+// in update_dir: x, the pool indices (scalar), the last W-1 steps, the weights.
+// Steps before those only move down by one. (One thread per channel and
+// 2-byte accesses before: 256 x 5120 bf16, W 4: 14.8 us, now 5.25, as lines of
+// W-1 take; S = 4 16.4 -> 5.7; W 9 26.5 -> 9.9; fp32 16.3 -> 9.2.)
+template <typename T, int W, int BPW, int WPG, bool SILU, bool HAS_BIAS, bool HAS_IDX>
+__global__ void __launch_bounds__(64 * WPG) update_step(const StepArgs<T> s) {
+    constexpr int H = W - 1;
+    constexpr int CPL = 4 / (int)sizeof(T);
+    const LinArgs<T>& a = s.l;
+    const int lane = threadIdx.x & 63;
+    const uint32_t cu = ((blockIdx.x * WPG + (threadIdx.x >> 6)) * 64u + lane) * CPL;
+    const bool on = cu < a.dim;
+    const uint32_t c = on ? cu : 0;  // lanes past the end read channel 0 and store nothing
+    const uint32_t b0 = blockIdx.y * BPW, nb = a.nbatch;
+    uint32_t xd[BPW];
+#pragma unroll
+    for (int q = 0; q < BPW; ++q)
+        xd[q] = __builtin_nontemporal_load(
+            reinterpret_cast<const uint32_t*>(a.x + (size_t)min(b0 + q, nb - 1) * a.x_row + c));
+    __builtin_amdgcn_sched_barrier(0);
+    int32_t row[BPW];
+#pragma unroll
+    for (int q = 0; q < BPW; ++q) {
+        const uint32_t b = min(b0 + q, nb - 1);
+        row[q] = HAS_IDX ? ld_uniform(a.idx + b) : (int32_t)b;
+        if (HAS_IDX && (row[q] < 0 || row[q] >= a.state_rows)) row[q] = -1;  // padding or out of the pool
+    }
+    uint32_t* sp[BPW];  // the lane's dword of step 0
+    const size_t step = s.state_step / CPL;
+    uint32_t st[BPW][H];
+#pragma unroll
+    for (int q = 0; q < BPW; ++q) {
+        sp[q] = reinterpret_cast<uint32_t*>(a.conv_state + (size_t)(row[q] >= 0 ? row[q] : 0) * a.state_row + c);
+#pragma unroll
+        for (int i = 0; i < H; ++i) st[q][i] = __builtin_nontemporal_load(sp[q] + (size_t)(s.S - H + i) * step);
+    }
+    uint32_t wd[W];  // CPL * W weights, raw
+    const uint32_t* wp = reinterpret_cast<const uint32_t*>(a.weight + (size_t)c * W);
+#pragma unroll
+    for (int k = 0; k < W; ++k) wd[k] = wp[k];
+    const uint32_t bd = HAS_BIAS ? *reinterpret_cast<const uint32_t*>(a.bias + c) : 0u;
+    __builtin_amdgcn_sched_barrier(0);  // every load is issued before any arithmetic
+    auto as_f32 = [](uint32_t d, int e) -> float {  // element e of a dword
+        if constexpr (CPL == 1) return __uint_as_float(d);
+        else return to_f32(T{(uint16_t)(e ? d >> 16 : d & 0xffffu)});
+    };
+#pragma unroll
+    for (int q = 0; q < BPW; ++q) {
+        float o[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < CPL; ++e) {
+            float win[W], w[W];
+#pragma unroll
+            for (int i = 0; i < H; ++i) win[i] = as_f32(st[q][i], e);
+            win[H] = as_f32(xd[q], e);
+#pragma unroll
+            for (int k = 0; k < W; ++k) w[k] = as_f32(wd[CPL == 1 ? k : (e * W + k) / 2], (e * W + k) & 1);
+            float acc = conv_taps<W>(HAS_BIAS ? as_f32(bd, e) : 0.0f, w, win);
+            if constexpr (SILU) acc = silu(acc);
+            o[e] = acc;
+        }
+        uint32_t od;
+        if constexpr (CPL == 1) od = __float_as_uint(o[0]);
+        else od = pack2<T>(o[0], o[1]);
+        if (row[q] < 0) od = 0u;  // padding entry: zero output, state untouched
+        if (!on || b0 + q >= nb) continue;  // (an entry past the batch computed on clamped data)
+        __builtin_nontemporal_store(od, reinterpret_cast<uint32_t*>(a.out + (size_t)(b0 + q) * a.out_row + c));
+        if (row[q] < 0) continue;
+        for (int i = 0; i + 1 < s.S - H; ++i) sp[q][(size_t)i * step] = sp[q][(size_t)(i + 1) * step];
+        if (s.S > H) __builtin_nontemporal_store(st[q][0], sp[q] + (size_t)(s.S - H - 1) * step);
+#pragma unroll
+        for (int i = 0; i < H; ++i)
+            __builtin_nontemporal_store(i + 1 < H ? st[q][i + 1 < H ? i + 1 : 0] : xd[q], sp[q] + (size_t)(s.S - H + i) * step);
     }
 }
 
@@ -807,11 +897,13 @@ template <typename T>
 bool lin_ok(const cc1d_update_params& p) {
     constexpr int64_t EPV = elems16<T>::value;
     const int64_t H = p.width - 1;
-    if (p.cache_seqlens != nullptr || p.seqlen != 1 || p.state_len != H) return false;
+    // (a state of W values instead of W-1 is common too: update_dir takes both;
+    // 256 x 5120 bf16, W 4: 16.9 us one thread per channel, 6.1 now)
+    if (p.cache_seqlens != nullptr || p.seqlen != 1 || (p.state_len != H && (p.state_len != H + 1 || H > 4))) return false;
     if (p.dim % EPV != 0) return false;
     if (p.x_stride[1] != 1 || p.out_stride[1] != 1) return false;
     if (p.x_stride[0] % EPV || p.out_stride[0] % EPV) return false;
-    if (p.conv_state_stride[2] != 1 || p.conv_state_stride[1] != H || p.conv_state_stride[0] % EPV) return false;
+    if (p.conv_state_stride[2] != 1 || p.conv_state_stride[1] != p.state_len || p.conv_state_stride[0] % EPV) return false;
     if (p.weight_stride[1] != 1 || p.weight_stride[0] != p.width) return false;
     if (p.bias != nullptr && (p.bias_stride != 1 || (reinterpret_cast<uintptr_t>(p.bias) & 3u))) return false;
     if (!aligned16(p.x) || !aligned16(p.out) || !aligned16(p.conv_state) ||
@@ -822,6 +914,27 @@ bool lin_ok(const cc1d_update_params& p) {
     if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim) return false;
     if (p.x_stride[0] >= lim || p.out_stride[0] >= lim || p.conv_state_stride[0] >= lim) return false;
     if (p.x_stride[0] < 0 || p.out_stride[0] < 0 || p.conv_state_stride[0] < 0) return false;
+    return true;
+}
+
+// unit channel stride of x, out and the state, whole dwords of channels
+template <typename T>
+bool step_ok(const cc1d_update_params& p) {
+    constexpr int64_t CPL = 4 / (int64_t)sizeof(T);
+    if (p.cache_seqlens != nullptr || p.seqlen != 1 || p.dim % CPL != 0) return false;
+    if (p.x_stride[1] != 1 || p.out_stride[1] != 1 || p.conv_state_stride[1] != 1) return false;
+    if (p.x_stride[0] % CPL || p.out_stride[0] % CPL || p.conv_state_stride[0] % CPL || p.conv_state_stride[2] % CPL)
+        return false;
+    if (p.weight_stride[1] != 1 || p.weight_stride[0] != p.width) return false;
+    if (p.bias != nullptr && (p.bias_stride != 1 || (reinterpret_cast<uintptr_t>(p.bias) & 3u))) return false;
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.out) |
+         reinterpret_cast<uintptr_t>(p.conv_state) | reinterpret_cast<uintptr_t>(p.weight)) & 3u)
+        return false;
+    // 32-bit channel indices and strides, a grid of (groups, batch) blocks; size_t offsets
+    const int64_t lim = (int64_t)1 << 31;
+    if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim || p.state_len >= lim) return false;
+    for (const int64_t st : {p.x_stride[0], p.out_stride[0], p.conv_state_stride[0], p.conv_state_stride[2]})
+        if (st < 0 || st >= lim) return false;
     return true;
 }
 
@@ -875,7 +988,8 @@ int launch_update(const cc1d_update_params& p, hipStream_t stream) {
                 constexpr bool SILU = decltype(sc)::value;
                 UpdArgs a;
                 a.p = p;
-                if (lin_ok<T>(p)) {
+                const bool lines = lin_ok<T>(p);
+                if (lines || step_ok<T>(p)) {
                     LinArgs<T> la;
                     la.x = static_cast<const T*>(p.x);
                     la.weight = static_cast<const T*>(p.weight);
@@ -889,13 +1003,29 @@ int launch_update(const cc1d_update_params& p, hipStream_t stream) {
                     la.dim = (uint32_t)p.dim;
                     la.state_rows = (int32_t)p.state_rows;
                     la.nbatch = (uint32_t)p.batch;
+                    if (!lines) {
+                        constexpr int CPL = 4 / (int)sizeof(T);
+                        const StepArgs<T> sa{la, (uint32_t)p.conv_state_stride[2], (int32_t)p.state_len};
+                        const dim3 gs((unsigned)ceil_div(ceil_div(p.dim, 64 * CPL), kDirWPG),
+                                      (unsigned)ceil_div(p.batch, kDirBPW));
+                        return with_flag(p.bias != nullptr, [&](auto hb) {
+                            return with_flag(p.conv_state_indices != nullptr, [&](auto hi) {
+                                return launch(update_step<T, W, kDirBPW, kDirWPG, SILU, decltype(hb)::value, decltype(hi)::value>,
+                                              gs, dim3(64 * kDirWPG), stream, sa);
+                            });
+                        });
+                    }
                     if constexpr (W - 1 <= 4) {
                         constexpr int CPL = 4 / (int)sizeof(T);
                         const dim3 gd((unsigned)ceil_div(ceil_div(p.dim, 64 * kDirNS * CPL), kDirWPG),
                                       (unsigned)ceil_div(p.batch, kDirBPW));
                         return with_flag(p.bias != nullptr, [&](auto hb) {
                             return with_flag(p.conv_state_indices != nullptr, [&](auto hi) {
-                                return launch(update_dir<T, W, kDirBPW, kDirNS, kDirWPG, SILU, decltype(hb)::value,
+                                if (p.state_len == W)
+                                    return launch(update_dir<T, W, W, kDirBPW, kDirNS, kDirWPG, SILU, decltype(hb)::value,
+                                                             decltype(hi)::value>,
+                                                  gd, dim3(64 * kDirWPG), stream, la);
+                                return launch(update_dir<T, W, W - 1, kDirBPW, kDirNS, kDirWPG, SILU, decltype(hb)::value,
                                                          decltype(hi)::value>,
                                               gd, dim3(64 * kDirWPG), stream, la);
                             });
