@@ -14,11 +14,14 @@
 // runs, which raises the errors and goes through the torch.library ops that
 // torch.compile, fake tensors, vmap, dispatch modes and the like see. The
 // backward asks again when it runs and goes through the same op if need be.
+// The interpreter lock is given up while a call allocates and launches: a
+// launch waits when the stream's queue is full, and other threads run on.
 // Nothing is kept from one call for the next.
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/dispatch/Dispatcher.h>
@@ -253,6 +256,7 @@ PyObject* py_fn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         return not_implemented();
     if (init.defined() && (!same(init, x) || !shaped(init, {B, D, W - 1}))) return not_implemented();
 
+    std::optional<pybind11::gil_scoped_release> unlocked(std::in_place);
     const c10::OptionalDeviceGuard device(x.device());
     auto wants = [](const Tensor& t) { return t.defined() && t.requires_grad(); };
     Tensor out, fs;
@@ -266,6 +270,7 @@ PyObject* py_fn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (final_states) fs = at::empty({B, D, W - 1}, x.options());
         launch_fwd(x, weight, bias, seq_idx, init, out, fs, act == 1);
     }
+    unlocked.reset();
     if (!final_states) return THPVariable_Wrap(std::move(out));
     PyObject* t = PyTuple_New(2);
     if (t == nullptr) throw python_error();
@@ -297,6 +302,7 @@ PyObject* py_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
                              !t->is_contiguous()))
             return not_implemented();
 
+    std::optional<pybind11::gil_scoped_release> unlocked(std::in_place);
     const c10::OptionalDeviceGuard device(x.device());
     Tensor out;
     {
@@ -327,6 +333,7 @@ PyObject* py_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
     p.dtype = dtype_code(x);
     p.apply_silu = act;
     check(api.update(&p, stream_of(x)));
+    unlocked.reset();
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -343,6 +350,7 @@ PyObject* py_varlen_states(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (over != 0 || S < 0 || x.dim() != 2 || cu.dim() != 1 || cu.size(0) < 1 || cu.scalar_type() != at::kInt ||
         cu.device() != x.device() || !cu.is_contiguous() || (es != 1 && es != 2 && es != 4 && es != 8 && es != 16))
         return not_implemented();
+    std::optional<pybind11::gil_scoped_release> unlocked(std::in_place);
     const c10::OptionalDeviceGuard device(x.device());
     Tensor states = at::empty({cu.size(0) - 1, S, x.size(1)}, x.options()).transpose(1, 2);
     cc1d_varlen_params p{};
@@ -358,6 +366,7 @@ PyObject* py_varlen_states(PyObject*, PyObject* const* a, Py_ssize_t n) {
     p.dtype = 0;
     p.elem_bytes = (int32_t)es;  // a bit-for-bit copy of any element type
     check(api.varlen(&p, stream_of(x)));
+    unlocked.reset();
     return THPVariable_Wrap(std::move(states));
     END_HANDLE_TH_ERRORS
 }
