@@ -748,8 +748,9 @@ __global__ void __launch_bounds__(256) update_circ_vec(const UpdArgs a) {
 // 16-byte chunks that change moves fewer bytes but costs more: with no
 // arithmetic, 256 x 5120 lines of 128 bytes take 62 us with one chunk of each
 // read and written (74 non-temporal), 49.7 with one granule (non-temporal;
-// 61 cached), 52.7 with the whole line. This kernel: C4b 53.8 us, 66.5 with
-// update_circ_vec. (Element places picked in registers instead of LDS, with
+// 61 cached), 52.7 with the whole line. This kernel: 53.8 us for those lines
+// (4 tokens), 66.5 with update_circ_vec; on random rows of a pool twice as
+// large 65.1 and 72.9. (Element places picked in registers instead of LDS, with
 // ds_bpermute and selects by wave-uniform indices, became 119 branches: 73 us.)
 template <typename T, int W, bool SILU, int NV>
 __global__ void __launch_bounds__(256) update_ring(const UpdArgs a) {
