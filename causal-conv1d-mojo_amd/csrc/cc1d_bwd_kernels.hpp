@@ -1592,8 +1592,10 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
             // 60.9 -> 50.0, 1023 40.1 -> 28.0, 511 23.8 -> 18.7; at ten times the batch
             // 575 -> 456, 350 -> 242, 191 -> 146). Otherwise alignment wins: unaligned
             // stores cost 7-20 % of a large fp32 or long-row call (fp32, batch 40,
-            // L = 2047: 850 -> 928; bf16 8 x 2048 x 16383: 272 -> 335).
-            if (sizeof(T) == 4 || pl.vpt * pl.a.nseg * 100 > vpt * nseg * 85) {
+            // L = 2047: 850 -> 928; bf16 8 x 2048 x 16383: 272 -> 335). Never for more
+            // segments: the workspace has a record for each of the aligned form's
+            // (384 vectors: 3 segments of 2 vectors per lane, 385: 2 of 4).
+            if (sizeof(T) == 4 || pl.vpt * pl.a.nseg * 100 > vpt * nseg * 85 || pl.a.nseg > nseg) {
                 pl.mode = kRowsAlike;
                 pl.vpt = vpt;
                 pl.a.nseg = nseg;
@@ -1652,8 +1654,9 @@ BwdPlan plan_bwd(const cc1d_bwd_params& p) {
 // of whole dwords of channels, else time chunks -- so that a size a program
 // has stored, or a problem that fits the static scratch, stays good when a
 // kernel takes more layouts or splits rows another way. Every plan's records
-// fit: kRowsShort has one per row, kRowsAny at most one per 64 steps, and
-// channels off the dword grid are only taken where they do.
+// fit: kRowsShort has one per row; kRowsAny at most one per 64 steps, and over
+// rows that lie alike no more than kRowsAlike's; channels off the dword grid are
+// only taken where they do. (plan_fits checks it before each launch.)
 template <typename T, int W>
 int64_t reserved_floats(const cc1d_bwd_params& p, const BwdPlan& pl) {
     constexpr int64_t EPV = elems16<T>::value;
@@ -1667,6 +1670,12 @@ int64_t reserved_floats(const cc1d_bwd_params& p, const BwdPlan& pl) {
     const int64_t rows = p.batch * p.dim;
     const int64_t nvec = aligned ? p.seqlen / EPV : ceil_div(p.seqlen + EPV - 1, EPV);
     return rows * ceil_div(nvec, 64 * (int64_t)rows_vpt(nvec, rows)) * pl.rec_floats;
+}
+
+// the workspace holds what the call asked for, and the records the plan writes
+template <typename T, int W>
+bool plan_fits(const cc1d_bwd_params& p, const BwdPlan& pl, int64_t workspace_floats) {
+    return reserved_floats<T, W>(p, pl) <= workspace_floats && pl.records * pl.rec_floats <= workspace_floats;
 }
 
 template <typename T, int W, bool SILU>
@@ -1861,7 +1870,7 @@ int launch_bwd_typed_dtype(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hi
         constexpr int W = decltype(wc)::value;
         return with_flag(p.apply_silu != 0, [&](auto sc) {
             BwdPlan pl = plan_bwd<T, W>(p);
-            if (reserved_floats<T, W>(p, pl) > g.workspace_floats) return (int)CC1D_ERR_WORKSPACE;
+            if (!plan_fits<T, W>(p, pl, g.workspace_floats)) return (int)CC1D_ERR_WORKSPACE;
             if (g.workspace == nullptr) return (int)CC1D_ERR_NULL_POINTER;
             pl.a.part = g.workspace;
             const int st = launch_plan<T, W, decltype(sc)::value>(pl, p, stream);

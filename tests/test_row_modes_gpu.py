@@ -6,10 +6,13 @@ memory around every row left as it was."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
 import causal_conv1d_amd as cc
+from causal_conv1d_amd import _lib, _native
 from _util import DTYPE_IDS, DTYPES, assert_close, assert_reduction_close, make_inputs, scales, seq_pattern
 from oracle import oracle as O
 
@@ -138,3 +141,33 @@ def test_nonfinite_rows_stay_with_their_row(dtype, activation, seqlen, mode):
     assert_close(out.detach().cpu()[:, keep], ref[:, keep], dtype)
     assert_close(xg.grad.cpu()[:, keep], rdx[:, keep], dtype)
     assert torch.equal(torch.isfinite(out.detach().cpu()), torch.isfinite(ref))
+
+
+@pytest.mark.parametrize("off", [0, 1])  # every tensor's first row, in elements past a 16-byte boundary
+@pytest.mark.parametrize("seqlen", [3066, 3071, 3072, 5114, 5119, 5120])
+def test_partial_sums_stay_in_the_workspace(seqlen, off):
+    """Lengths whose vectors, counted from a row's first element and from the 16-byte boundary
+    before it, are split into another number of segments: the floats behind the workspace
+    stay as they were, and the sums are right."""
+    B, D, W, dtype = 2, 48, 4, torch.bfloat16
+    x, w, b, _ = make_inputs(B, D, seqlen, W, dtype=dtype)
+    dout = make_inputs(B, D, seqlen, W, dtype=dtype, seed=1)[0]
+    (xg, _), (gg, _), (dg, _) = (_rows(t, off, 0) for t in (x, dout, torch.zeros_like(x)))
+    wg, bg = w.to(DEV), b.to(DEV)
+    dw, db = torch.empty_like(wg), torch.empty_like(bg)
+    p = _native._bwd_params(xg, wg, bg, gg, None, None, dg, None, True, None)
+    lib = _lib.load()
+    n = lib.cc1d_bwd_workspace_floats(ctypes.byref(p))
+    ws = torch.full((2 * n,), GUARD, device=DEV)
+    g = _lib.BwdGrads()
+    g.dweight, g.dbias, g.workspace, g.workspace_floats = dw.data_ptr(), db.data_ptr(), ws.data_ptr(), n
+    g.dweight_stride[:] = (W, 1)
+    g.dbias_stride = 1
+    assert lib.cc1d_bwd_typed(ctypes.byref(p), ctypes.byref(g), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool((ws[n:] == GUARD).all())
+    rdx, rdw, rdb, _ = O.causal_conv1d_bwd(x, w, b, dout, activation="silu")
+    assert_close(dg.cpu(), rdx, dtype)
+    sw, sb = scales(x, w, b, dout, activation="silu")
+    assert_reduction_close(dw.cpu(), rdw, dtype, scale=sw, name="dweight")
+    assert_reduction_close(db.cpu(), rdb, dtype, scale=sb, name="dbias")
