@@ -254,6 +254,13 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
         const int wl = SHORT ? (int)(threadIdx.x & 63) : lane;  // lane of the wavefront
         const int prev_lane = (wl + 63) & 63;
         const int next_lane = (wl + 1) & 63;
+        // Without initial_states a tap that reaches before the row adds no
+        // weight-gradient term (a select: zero times a non-finite dpre would be
+        // NaN; C2's shape, rows unlike, L = 2041: 47.3 us without, 47.7). In the
+        // aligned modes the selects cost a wavefront per SIMD (96 registers), so
+        // those add the product with zero.
+        constexpr bool UNALIGNED = MODE == kRowsAny || SHORT;
+        const bool row_head = lane == 0 && t0 == 0 && p.initial_states == nullptr;
 
         // ---- dpre of vector j + dweight/dbias partials ----
         // PART: some lane's vector j may hold a position outside the row
@@ -303,7 +310,8 @@ __device__ __forceinline__ void bwd_rows_compute(const cc1d_bwd_params& p, int l
 #pragma unroll
                 for (int k = 0; k < W; ++k) {
                     const float s = __builtin_fmaf(d, win[i + k], pw[k]);
-                    pw[k] = (EDGES && outside) ? pw[k] : s;
+                    const bool before = UNALIGNED && j == 0 && i + k < H && row_head;
+                    pw[k] = ((EDGES && outside) || before) ? pw[k] : s;
                 }
             }
         };
@@ -607,14 +615,20 @@ __device__ __forceinline__ void bwd_rows_compute_seq(const cc1d_bwd_params& p, i
             // whatever the row holds
             if (cur < 0) d = 0.0f;
             pb += d;
+            // a tap that is not kept adds no term to the weight gradient, and none
+            // to dx: both take its dpre as zero (times the zero x above), so that a
+            // non-finite dpre stays with the taps it has
+            float de[W];
 #pragma unroll
-            for (int kk = 0; kk < W; ++kk) pw[kk] = __builtin_fmaf(d, xe[kk], pw[kk]);
+            for (int kk = 0; kk < W; ++kk) {
+                de[kk] = keep[kk] ? d : 0.0f;
+                pw[kk] = __builtin_fmaf(de[kk], xe[kk], pw[kk]);
+            }
             // dx[s - k] += w[W-1-k] * dpre[s] where tap W-1-k of s is kept
 #pragma unroll
             for (int k = 0; k <= H; ++k) {
-                const float de = keep[H - k] ? d : 0.0f;
-                if (e - k >= 0) a[e - k] = __builtin_fmaf(w[W - 1 - k], de, a[e - k]);
-                else cr[H + e - k] = __builtin_fmaf(w[W - 1 - k], de, cr[H + e - k]);
+                if (e - k >= 0) a[e - k] = __builtin_fmaf(w[W - 1 - k], de[H - k], a[e - k]);
+                else cr[H + e - k] = __builtin_fmaf(w[W - 1 - k], de[H - k], cr[H + e - k]);
             }
             // one position at a time: the sums are updated here (the compiler
             // would otherwise sink their fmas to the end, keeping every

@@ -171,3 +171,42 @@ def test_partial_sums_stay_in_the_workspace(seqlen, off):
     sw, sb = scales(x, w, b, dout, activation="silu")
     assert_reduction_close(dw.cpu(), rdw, dtype, scale=sw, name="dweight")
     assert_reduction_close(db.cpu(), rdb, dtype, scale=sb, name="dbias")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DTYPE_IDS)
+@pytest.mark.parametrize("place", list(PLACES))
+@pytest.mark.parametrize("activation", [None, "silu"])
+@pytest.mark.parametrize("seqlen", [2, 21, 64, 261, 1021, 2051])
+@pytest.mark.parametrize("where", ["row", "sequence"])
+def test_nonfinite_dout_stays_with_the_taps_it_has(dtype, place, activation, seqlen, where):
+    """dout of channel 6 is NaN at its row's first position, or at the first position of the row's
+    second sequence: the reference adds no term there for the taps before (bwd_full_cpu/
+    kernel.mojo:264-274), so only the channel's last tap and its bias are NaN. (Rows of more than
+    32 vectors that lie alike take aligned vectors, which add a product with zero at a row's start:
+    test_ragged_gpu.py's expected failures.)"""
+    if where == "row" and place != "unlike" and seqlen > 64:
+        pytest.skip("aligned vectors")
+    B, D, W = 2, 12, 4
+    x, w, b, _ = make_inputs(B, D, seqlen, W, dtype=dtype)
+    dout = make_inputs(B, D, seqlen, W, dtype=dtype, seed=1)[0]
+    seq = None
+    if where == "sequence":
+        seq = torch.zeros(B, seqlen, dtype=torch.int32)
+        seq[:, seqlen // 2:] = 1
+    dout[:, 6, 0 if seq is None else seqlen // 2] = float("nan")
+    (px, po, pg) = PLACES[place]
+    (xg, _), (gg, _), (dg, _) = _rows(x, *px), _rows(dout, *pg), _rows(torch.zeros_like(x), *po)
+    wg, bg = w.to(DEV), b.to(DEV)
+    dw, db = torch.empty_like(wg), torch.empty_like(bg)
+    torch.ops.causal_conv1d_amd._bwd_typed_inplace(xg, wg, bg, gg, None if seq is None else seq.to(DEV), None, None, dg,
+                                                   dw, db, None, activation is not None)
+    rdx, rdw, rdb, _ = O.causal_conv1d_bwd(x, w, b, dout, seq_idx=seq, activation=activation)
+    sw, sb = scales(x, w, b, torch.nan_to_num(dout), seq_idx=seq, activation=activation)
+    assert int((~torch.isfinite(rdw.double())).sum()) == 1, "the case is what it says"
+    for got, want, scale in ((dg, rdx, None), (dw, rdw, sw), (db, rdb, sb)):
+        got, fin = got.cpu(), torch.isfinite(want.double())
+        assert torch.equal(torch.isfinite(got.double()), fin)
+        if scale is None:
+            assert_close(got[fin], want[fin], dtype)
+        else:
+            assert_reduction_close(got[fin], want[fin], dtype, scale=scale[fin])
