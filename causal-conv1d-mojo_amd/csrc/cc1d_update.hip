@@ -910,9 +910,10 @@ bool lin_ok(const cc1d_update_params& p) {
     if (!aligned16(p.x) || !aligned16(p.out) || !aligned16(p.conv_state) ||
         (reinterpret_cast<uintptr_t>(p.weight) & 3u))
         return false;
-    // 32-bit channel indices and row strides, a grid of (groups, batch) blocks; size_t offsets
+    // 32-bit channel indices and row strides, a grid of (groups, batch) blocks; size_t
+    // offsets; a row 0 for padding entries to read
     const int64_t lim = (int64_t)1 << 31;
-    if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim) return false;
+    if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim || p.state_rows < 1) return false;
     if (p.x_stride[0] >= lim || p.out_stride[0] >= lim || p.conv_state_stride[0] >= lim) return false;
     if (p.x_stride[0] < 0 || p.out_stride[0] < 0 || p.conv_state_stride[0] < 0) return false;
     return true;
@@ -931,9 +932,9 @@ bool step_ok(const cc1d_update_params& p) {
     if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.out) |
          reinterpret_cast<uintptr_t>(p.conv_state) | reinterpret_cast<uintptr_t>(p.weight)) & 3u)
         return false;
-    // 32-bit channel indices and strides, a grid of (groups, batch) blocks; size_t offsets
+    // as in lin_ok
     const int64_t lim = (int64_t)1 << 31;
-    if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim || p.state_len >= lim) return false;
+    if (p.dim >= lim || p.batch > 65535 || p.state_rows >= lim || p.state_rows < 1 || p.state_len >= lim) return false;
     for (const int64_t st : {p.x_stride[0], p.out_stride[0], p.conv_state_stride[0], p.conv_state_stride[2]})
         if (st < 0 || st >= lim) return false;
     return true;

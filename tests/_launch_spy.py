@@ -133,4 +133,23 @@ def floats_touched():
     return wrote, read
 
 
-__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "ctypes", "_lib", "FAKE"]
+def update(B, D, W, dtype, *, S, state="line", rows=None, tokens=1, ring=False, indices=False):
+    """Kernel of a decode update: state rows of lines (a channel's S values together) or steps."""
+    launches.clear()
+    p = _lib.UpdateParams()
+    p.x, p.weight, p.bias, p.conv_state, p.out = (FAKE,) * 5
+    p.conv_state_indices = FAKE if indices else None
+    p.cache_seqlens = FAKE if ring else None
+    p.batch, p.dim, p.seqlen, p.width, p.state_len = B, D, tokens, W, S
+    p.state_rows = B if rows is None else rows
+    p.x_stride[:] = p.out_stride[:] = (D * tokens, tokens, 1)
+    p.weight_stride[:] = (W, 1)
+    p.bias_stride = 1
+    p.conv_state_stride[:] = (D * S, S, 1) if state == "line" else (D * S, 1, D)
+    p.dtype, p.apply_silu = dtype, 1
+    status = lib.cc1d_update(ctypes.byref(p), None)
+    assert status == 0 and len(launches) == 1, status
+    return launches[0][0]
+
+
+__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "update", "ctypes", "_lib", "FAKE"]

@@ -67,3 +67,17 @@ result = {"kinds": kinds, "bad": bad[:40], "n_bad": len(bad), "scratch": scratch
     assert set(got["kinds"]) == {"bwd_rows_vec", "bwd_rows_short", "bwd_clw", "bwd_generic"}, got["kinds"]
     assert got["n_bad"] == 0, got["bad"]
     assert got["scratch"] == [[0, 2_000_000], [9, 0]]  # CC1D_ERR_SCRATCH_LIMIT past 2,097,152
+
+
+def test_an_empty_pool_takes_a_kernel_that_reads_no_row(tmp_path):
+    """With no row in the pool every index is padding; update_dir, update_lin and update_step
+    read row 0 in a padding entry's place, so such calls go to the generic kernel."""
+    code = r"""
+result = []
+for dtype in (0, 1, 2):
+    for W, S, state in ((4, 3, "line"), (4, 4, "line"), (9, 8, "line"), (4, 3, "step"), (9, 8, "step"), (4, 6, "step")):
+        result.append([update(3, 64, W, dtype, S=S, state=state, rows=r, indices=True) for r in (5, 0)])
+"""
+    got = _launch_spy.run(code, tmp_path)
+    assert {a for a, _ in got} == {"update_dir", "update_lin", "update_step"}
+    assert {b for _, b in got} == {"update_generic"}
