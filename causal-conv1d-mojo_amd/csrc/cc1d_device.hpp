@@ -375,6 +375,17 @@ __device__ __forceinline__ int32_t lane_get(int32_t v, int src) {
     return __builtin_amdgcn_ds_bpermute(src << 2, v);
 }
 
+// Between LDS writes and reads of one wavefront's lanes: what any lane wrote
+// before is what every lane reads after. A wavefront's LDS accesses complete in
+// order, so the fences cost no instruction; they keep the compiler, to which the
+// lanes are separate threads, from moving or forwarding an access across (a wave
+// barrier alone orders no memory).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // DPP controls (GFX9 encoding) for the wavefront reduction below.
 constexpr int kDppQuadSwap1 = 0xb1;   // quad_perm [1, 0, 3, 2]
 constexpr int kDppQuadSwap2 = 0x4e;   // quad_perm [2, 3, 0, 1]

@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(64) update_lin(const LinArgs<T> a) {
         if (64 * j + 63 >= NSV) v = vi >= NSV ? xv[j] : v;
         seg[64 * j + lane] = v;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     uint32_t* sd = reinterpret_cast<uint32_t*>(seg);
     uint32_t st[SD], xd[XD];
 #pragma unroll
@@ -264,12 +264,12 @@ __global__ void __launch_bounds__(64) update_lin(const LinArgs<T> a) {
             for (int i = 0; i < XD; ++i) od[i] = 0u;
         }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
 #pragma unroll
     for (int i = 0; i < SD; ++i) sd[SD * lane + i] = nd[i];
 #pragma unroll
     for (int i = 0; i < XD; ++i) sd[4 * NSV + XD * lane + i] = od[i];
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     T* orow = a.out + (size_t)b * a.out_row + c0;
 #pragma unroll
     for (int j = 0; j < NSLOT; ++j) {
@@ -837,14 +837,14 @@ __global__ void __launch_bounds__(256) update_ring(const UpdArgs a) {
         *reinterpret_cast<u32x4*>(g) = va[i];
         if (two) *reinterpret_cast<u32x4*>(g + GRB) = vb[i];
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     // (the W-1 + Ls window positions are distinct: ring_ok keeps them within S)
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         if (q < Ls) *at(i, O + H + q) = xt[i][0];
         if (q + 4 < Ls) *at(i, O + H + q + 4) = xt[i][1];
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         float w[W];
