@@ -1030,7 +1030,7 @@ template <typename T> __device__ __forceinline__ void row_store_nt(T* base, uint
 // the block adds the sums with fp32 atomics on consecutive addresses (or
 // writes them as its record). Block order: channel group fastest, then run
 // group, then batch.
-template <typename T, int W, int G, int R, int WPB, bool SILU, bool SEQ>
+template <typename T, int W, int G, int R, int WPB, bool SILU, bool SEQ, bool ODD>
 __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
     constexpr int CPL = 4 / (int)sizeof(T);
     constexpr int H = W - 1;
@@ -1054,12 +1054,13 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
     const int32_t t0 = (int32_t)uniform32((tg * WPB + wave) * R);
     const int32_t cw0 = (int32_t)(grp * NC);
     const bool active = cw0 + lane * CPL < (int32_t)p.dim;
-    // the last lane of an odd number of 16-bit channels takes the last CPL ones
-    // (`shifted`): the channel it shares with the lane before gets the same dx
-    // from both, and its share of the sums is dropped below. cb: the channel
+    // ODD: the last lane of an odd number of 16-bit channels takes the last CPL
+    // ones (`shifted`): the channel it shares with the lane before gets the same
+    // dx from both, and its share of the sums is dropped below. cb: the channel
     // the wavefront's row addresses start from
-    const int32_t cb = cw0 + CPL <= (int32_t)p.dim ? cw0 : (int32_t)p.dim - CPL;
-    const bool shifted = active && cw0 + lane * CPL + CPL > (int32_t)p.dim;
+    static_assert(!ODD || CPL == 2, "a lane's channels can only be cut in two");
+    const int32_t cb = !ODD || cw0 + CPL <= (int32_t)p.dim ? cw0 : (int32_t)p.dim - CPL;
+    const bool shifted = ODD && active && cw0 + lane * CPL + CPL > (int32_t)p.dim;
     const int32_t c0 = shifted ? (int32_t)p.dim - CPL : cw0 + lane * CPL;
 
     ClWalk<W, CPL> s;
@@ -1368,7 +1369,7 @@ __global__ void __launch_bounds__(64 * WPB) bwd_clw(const BwdArgs a) {
                 for (int k = 0; k < W; ++k) s.pw[k][e] = 0.0f;
             }
         }
-        if constexpr (CPL == 2) {
+        if constexpr (ODD) {
             if (shifted) {  // the last channel's sums go to its own place, the lane's first
                 s.pb[0] = s.pb[1];
                 s.pb[1] = 0.0f;
@@ -1720,9 +1721,21 @@ int launch_plan(const BwdPlan& pl, const cc1d_bwd_params& p, hipStream_t stream)
             constexpr bool SEQ = decltype(qc)::value;
             constexpr int G = W - 1 <= kClG ? kClG : 2 * kClG;  // at least H steps per chunk
             const dim3 block(64 * kClWPB);
-            if (a.chunk == kClRShort) return launch(bwd_clw<T, W, G, kClRShort, kClWPB, SILU, SEQ>, grid, block, stream, a);
-            if (a.chunk == kClRMid) return launch(bwd_clw<T, W, G, kClRMid, kClWPB, SILU, SEQ>, grid, block, stream, a);
-            return launch(bwd_clw<T, W, G, kClR, kClWPB, SILU, SEQ>, grid, block, stream, a);
+            auto go = [&](auto oc) {
+                constexpr bool ODD = decltype(oc)::value;
+                if (a.chunk == kClRShort)
+                    return launch(bwd_clw<T, W, G, kClRShort, kClWPB, SILU, SEQ, ODD>, grid, block, stream, a);
+                if (a.chunk == kClRMid)
+                    return launch(bwd_clw<T, W, G, kClRMid, kClWPB, SILU, SEQ, ODD>, grid, block, stream, a);
+                return launch(bwd_clw<T, W, G, kClR, kClWPB, SILU, SEQ, ODD>, grid, block, stream, a);
+            };
+            constexpr int CPL = 4 / (int)sizeof(T);
+            if constexpr (CPL == 1) return go(std::false_type{});
+            // the odd count's addresses cost whole dwords of channels scalar registers
+            // (seq_idx at W 4: 44 scalar spills, 43 without them; us at 1 x 4096 x
+            // 8192 bf16, one form for all -> two: seq_idx 39.8 -> 39.4, with the
+            // reduction 42.4 -> 41.9; plain 37.9 -> 37.8)
+            else return with_flag(!cl_dwords<T, CPL>(p), go);
         });
     }
     return launch(bwd_generic<T, W, SILU>, grid, dim3(256), stream, a);

@@ -49,7 +49,7 @@ class RedArgs(ctypes.Structure):
 
 
 lib = None
-launches: list = []  # (kernel, grid x, grid y, block x, struct of its argument or None, RowsMode)
+launches: list = []  # (kernel, grid x, grid y, block x, struct of its argument or None, mangled name)
 _keep: list = []
 
 
@@ -59,10 +59,9 @@ def _name(mangled: str) -> str:
     return mangled[m.end():m.end() + int(m.group(1))]
 
 
-def _mode(mangled: str) -> int:
-    """The last integer template argument (the RowsMode of the *_rows_vec kernels)."""
-    found = re.findall(r"Li(\d+)E", mangled)
-    return int(found[-1]) if found else -1
+def template_values(mangled: str) -> list[int]:
+    """The integer and boolean template arguments, in order."""
+    return [int(v) for v in re.findall(r"L[ib](\d+)E", mangled)]
 
 
 def setup(spy_path: str) -> None:
@@ -78,7 +77,7 @@ def setup(spy_path: str) -> None:
             arg = RedArgs.from_buffer_copy(ctypes.string_at(args[0], ctypes.sizeof(RedArgs)))
         elif kernel.startswith("bwd_"):
             arg = BwdArgs.from_buffer_copy(ctypes.string_at(args[0], ctypes.sizeof(BwdArgs)))
-        launches.append((kernel, gx, gy, bx, arg, _mode(mangled)))
+        launches.append((kernel, gx, gy, bx, arg, mangled))
 
     _keep.extend((spy, cb_type(on_launch)))
     spy.spy_callback(_keep[-1])
@@ -152,4 +151,5 @@ def update(B, D, W, dtype, *, S, state="line", rows=None, tokens=1, ring=False, 
     return launches[0][0]
 
 
-__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "update", "ctypes", "_lib", "FAKE"]
+__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "template_values", "update",
+           "ctypes", "_lib", "FAKE"]

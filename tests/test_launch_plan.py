@@ -81,3 +81,20 @@ for dtype in (0, 1, 2):
     got = _launch_spy.run(code, tmp_path)
     assert {a for a, _ in got} == {"update_dir", "update_lin", "update_step"}
     assert {b for _, b in got} == {"update_generic"}
+
+
+def test_channel_last_rows_of_whole_dwords_keep_their_own_kernel(tmp_path):
+    """An even number of 16-bit channels on the dword grid takes the form of bwd_clw without the
+    odd count's addresses (its last template argument), anything else the one with them."""
+    code = r"""
+result = []
+for dtype, D, kw in ((1, 768, {}), (0, 4096, {}), (1, 769, {}), (1, 768, dict(dim_pad=1)), (0, 768, dict(offsets=(0, 2, 0))),
+                     (2, 769, {})):
+    for seq in (None, 1):
+        p = bwd_params(2, D, 512, 4, dtype, layout="last", seq_stride=seq, **kw)
+        assert bwd_typed(p) == 0
+        result.append([launches[0][0], template_values(launches[0][5])[-1]])
+"""
+    got = _launch_spy.run(code, tmp_path)
+    assert {k for k, _ in got} == {"bwd_clw"}
+    assert [odd for _, odd in got] == [0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 0, 0]
