@@ -4,8 +4,13 @@ call that something observes or transforms goes through the ops as before."""
 
 from __future__ import annotations
 
+import threading
+
 import pytest
 import torch
+import torch.utils.checkpoint
+from functorch.compile import make_boxed_func
+from torch._dynamo.backends.common import aot_autograd
 from torch.utils._python_dispatch import TorchDispatchMode
 
 import causal_conv1d_amd as cc
@@ -216,3 +221,120 @@ def test_errors_as_before():
         cc.causal_conv1d_fn(x, kw["weight"].cpu())
     with pytest.raises(ValueError, match="must be >="):
         cc.causal_conv1d_update(x[..., 0], torch.zeros(B, D, 2, device=DEV, dtype=x.dtype), kw["weight"])
+
+
+def _step(x, kw, dout):
+    """Fresh leaves, one training step: (out, dx, dweight, dbias)."""
+    xs = x.detach().clone().requires_grad_()
+    w, b = (kw[k].detach().clone().requires_grad_() for k in ("weight", "bias"))
+    out = cc.causal_conv1d_fn(xs, w, b, activation="silu")
+    return [out.detach(), *torch.autograd.grad(out, [xs, w, b], dout)]
+
+
+def test_threads_each_on_a_stream_of_its_own():
+    """The lock is given up while a call allocates and launches: calls of several threads interleave."""
+    x, kw = _args("plain")
+    douts = [torch.randn_like(x).detach() for _ in range(4)]
+    want = [_step(x, kw, g) for g in douts]
+    got, errors = {}, []
+    torch.cuda.synchronize()
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                got[i] = [_step(x, kw, douts[i]) for _ in range(20)]
+                torch.cuda.current_stream().synchronize()
+        except BaseException as e:  # noqa: BLE001 -- reported below
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors and len(got) == 4
+    for i, runs in got.items():
+        assert all(torch.equal(a, b) for run in runs for a, b in zip(run, want[i], strict=True))
+
+
+def test_calls_follow_the_current_stream():
+    """Inputs made late on a side stream: forward there, backward from outside the block."""
+    x, kw = _args("plain")
+    dout = torch.randn_like(x).detach()
+    want = _step(x, kw, dout)
+    state = torch.randn(B, D, W - 1, device=DEV).to(x.dtype)
+    tok = x.detach()[..., 0].contiguous()
+    ref_state = state.clone()
+    ref_tok = cc.causal_conv1d_update(tok, ref_state, kw["weight"].detach())
+    big = torch.randn(4096, 4096, device=DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        late = torch.zeros_like(x.detach())
+        for _ in range(8):
+            big = big @ big * 1e-3  # the inputs arrive after this
+        late.copy_(x.detach())
+        late.requires_grad_()
+        w, b = (kw[k].detach().clone().requires_grad_() for k in ("weight", "bias"))
+        out = cc.causal_conv1d_fn(late, w, b, activation="silu")
+        own = state.clone()
+        step = cc.causal_conv1d_update(late.detach()[..., 0].contiguous(), own, w.detach())
+    torch.cuda.current_stream().wait_stream(side)
+    grads = torch.autograd.grad(out, [late, w, b], dout)
+    torch.cuda.synchronize()
+    for a, c in zip([out.detach(), *grads, step, own], [*want, ref_tok, ref_state], strict=True):
+        assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("reentrant", [True, False])
+def test_activation_checkpointing(reentrant):
+    x, kw = _args("plain")
+    dout = torch.randn_like(x).detach()
+    want = _step(x, kw, dout)
+    xs = x.detach().clone().requires_grad_()
+    w, b = (kw[k].detach().clone().requires_grad_() for k in ("weight", "bias"))
+
+    def f(t):
+        return cc.causal_conv1d_fn(t, w, b, activation="silu")
+
+    out = torch.utils.checkpoint.checkpoint(f, xs, use_reentrant=reentrant)
+    out.backward(dout)
+    for a, c in zip([out.detach(), xs.grad, w.grad, b.grad], want, strict=True):
+        assert torch.equal(a, c)
+
+
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")  # torch's own, on importing its compiler
+@pytest.mark.parametrize("mode", ["plain", "seq", "states", "nobias"])
+@pytest.mark.parametrize("how", ["run", "compile"])
+def test_compiled_autograd(mode, how):
+    """A backward captured as a graph, with the native node as a call of its own in it: run as it
+    is, and traced and compiled further, where the node's backward goes through the op."""
+    from torch._dynamo import compiled_autograd
+
+    x, kw = _args(mode)
+    dout = torch.randn_like(x).detach()
+    dfinal = torch.randn(B, D, W - 1, device=DEV).to(x.dtype)
+    want = _run(x, kw, dout, dfinal)
+    captured, traced = [], []
+    torch._dynamo.reset()  # (a backward captured before would be taken again)
+    torch._C._dynamo.compiled_autograd.clear_cache()
+
+    def note(gm, inputs):
+        traced.extend(f"{n.target} {n.args}" for n in gm.graph.nodes)
+        return make_boxed_func(gm.forward)
+
+    def compiler(gm):
+        captured.extend(str(n.target) for n in gm.graph.nodes)
+        return gm if how == "run" else torch.compile(gm, backend=aot_autograd(fw_compiler=note))
+
+    r = cc.causal_conv1d_fn(x, **kw)
+    out, final = r if isinstance(r, tuple) else (r, None)
+    ins = [t for t in (x, kw["weight"], kw["bias"], kw.get("initial_states")) if t is not None]
+    outs, douts = ([out, final], [dout, dfinal]) if final is not None else ([out], [dout])
+    with compiled_autograd._enable(compiler):
+        torch.autograd.backward(outs, douts)
+    got = [out, *([final] if final is not None else []), *(t.grad for t in ins)]
+    assert any("Conv1dFn" in t for t in captured)
+    assert how == "run" or any("_bwd_typed_inplace" in t for t in traced)
+    for a, c in zip(got, want, strict=True):
+        assert torch.equal(a.detach(), c.detach())
