@@ -84,6 +84,14 @@ def setup(spy_path: str) -> None:
     lib = _lib.load()
 
 
+def _strides(layout, D, L, pad, dim_pad):
+    if layout == "rows":
+        return D * (L + pad), L + pad, 1
+    if layout == "last":
+        return L * (D + dim_pad), 1, D + dim_pad
+    return 2 * D * L, 2 * L, 2  # no unit stride
+
+
 def bwd_params(B, D, L, W, dtype, *, layout="rows", offsets=(0, 0, 0), pads=(0, 0, 0), seq_stride=None, dim_pad=0):
     """cc1d_bwd_params of tensors that lie as said: byte offsets and row pads (elements) of x, dout and dx."""
     p = _lib.BwdParams()
@@ -91,12 +99,7 @@ def bwd_params(B, D, L, W, dtype, *, layout="rows", offsets=(0, 0, 0), pads=(0, 
     p.weight, p.bias = FAKE, FAKE
     p.batch, p.dim, p.seqlen, p.width, p.dtype, p.apply_silu = B, D, L, W, dtype, 1
     for stride, pad in zip((p.x_stride, p.dout_stride, p.dx_stride), pads):
-        if layout == "rows":
-            stride[:] = (D * (L + pad), L + pad, 1)
-        elif layout == "last":
-            stride[:] = (L * (D + dim_pad), 1, D + dim_pad)
-        else:  # no unit stride
-            stride[:] = (2 * D * L, 2 * L, 2)
+        stride[:] = _strides(layout, D, L, pad, dim_pad)
     p.weight_stride[:] = (W, 1)
     p.bias_stride = 1
     if seq_stride is not None:
@@ -132,6 +135,30 @@ def floats_touched():
     return wrote, read
 
 
+def fwd(B, D, L, W, dtype, *, layout="rows", offsets=(0, 0), pads=(0, 0), seq=False, dim_pad=0):
+    """Kernel of a forward, and its RowsMode (None unless fwd_rows_vec)."""
+    launches.clear()
+    p = _lib.FwdParams()
+    p.x, p.out = (FAKE + o for o in offsets)
+    p.weight, p.bias = FAKE, FAKE
+    p.batch, p.dim, p.seqlen, p.width, p.dtype, p.apply_silu = B, D, L, W, dtype, 1
+    for stride, pad in zip((p.x_stride, p.out_stride), pads):
+        stride[:] = _strides(layout, D, L, pad, dim_pad)
+    p.weight_stride[:] = (W, 1)
+    p.bias_stride = 1
+    if seq:
+        p.seq_idx = FAKE
+        p.seq_idx_stride[:] = (L, 1)
+    status = lib.cc1d_fwd(ctypes.byref(p), None)
+    assert status == 0 and len(launches) == 1, status
+    return route(launches[0])
+
+
+def route(launch):
+    """[kernel, RowsMode of a *_rows_vec kernel or None]"""
+    return [launch[0], template_values(launch[5])[-1] if launch[0].endswith("rows_vec") else None]
+
+
 def update(B, D, W, dtype, *, S, state="line", rows=None, tokens=1, ring=False, indices=False):
     """Kernel of a decode update: state rows of lines (a channel's S values together) or steps."""
     launches.clear()
@@ -151,5 +178,5 @@ def update(B, D, W, dtype, *, S, state="line", rows=None, tokens=1, ring=False, 
     return launches[0][0]
 
 
-__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "template_values", "update",
+__all__ = ["lib", "launches", "bwd_params", "bwd_typed", "floats_touched", "template_values", "route", "fwd", "update",
            "ctypes", "_lib", "FAKE"]

@@ -226,11 +226,12 @@ def test_workspace_sizes_of_the_benchmark_configurations(lib):
     assert max(sizes.values()) <= _lib.NOALLOC_WORKSPACE_FLOATS == 2_097_152
 
 
-def test_ragged_rows_keep_the_row_kernel(lib):
+def test_workspace_sizes_of_ragged_rows(lib):
     """Rows whose length is not a multiple of the 16-byte vector, or that start off a 16-byte
-    boundary, are planned as row segments (one record of W + 1 floats per segment of 64 lanes
-    x VPT vectors, spanning ceil((L + EPV - 1) / EPV) vectors); the generic kernel would take
-    64-step chunks. dout or dx at another offset modulo 16 bytes falls back to it."""
+    boundary, are sized as row segments (one record of W + 1 floats per segment of 64 lanes
+    x VPT vectors, spanning ceil((L + EPV - 1) / EPV) vectors), tensors that lie unlike each other
+    and strided ones as 64-step chunks. The sizes depend on lengths and layout alone, not on the
+    kernel that runs (test_launch_plan.py has that, and that its records fit)."""
     B, D, W = 1, 64, 4
 
     def rows(L, epv, aligned=False, B=B, D=D):
@@ -242,7 +243,7 @@ def test_ragged_rows_keep_the_row_kernel(lib):
             vpt = 2  # the last 4-vector segment would be mostly empty
         return B * D * -(-nvec // (64 * vpt)) * (W + 1)
 
-    def generic(L):
+    def chunks(L):
         return B * D * -(-L // 64) * (W + 1)
 
     bf16, fp32 = 1, 2
@@ -256,9 +257,9 @@ def test_ragged_rows_keep_the_row_kernel(lib):
     # a base one element past a 16-byte boundary, x / dout / dx alike
     assert _workspace_floats(lib, B, D, 2048, bf16, offsets=(2, 2, 2)) == rows(2048, 8) == 960
     assert _workspace_floats(lib, B, D, 2048, fp32, offsets=(4, 4, 4)) == rows(2048, 4) == 1600
-    # dout at another offset inside its vector than x: the generic kernel
-    assert _workspace_floats(lib, B, D, 2047, bf16, offsets=(0, 2, 0)) == generic(2047) == 10240
-    assert _workspace_floats(lib, B, D, 2048, bf16, offsets=(2, 2, 4)) == generic(2048) == 10240
-    # seq_idx: unit time stride keeps the row kernel; the ragged id loads need it, others go generic
+    # dout at another offset inside its vector than x
+    assert _workspace_floats(lib, B, D, 2047, bf16, offsets=(0, 2, 0)) == chunks(2047) == 10240
+    assert _workspace_floats(lib, B, D, 2048, bf16, offsets=(2, 2, 4)) == chunks(2048) == 10240
+    # seq_idx: with a unit time stride as without ids; other strides as chunks (the generic kernel)
     assert _workspace_floats(lib, B, D, 2047, bf16, seq_stride=1) == rows(2047, 8) == 960
-    assert _workspace_floats(lib, B, D, 2047, bf16, seq_stride=2) == generic(2047) == 10240
+    assert _workspace_floats(lib, B, D, 2047, bf16, seq_stride=2) == chunks(2047) == 10240

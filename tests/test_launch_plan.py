@@ -98,3 +98,53 @@ for dtype, D, kw in ((1, 768, {}), (0, 4096, {}), (1, 769, {}), (1, 768, dict(di
     got = _launch_spy.run(code, tmp_path)
     assert {k for k, _ in got} == {"bwd_clw"}
     assert [odd for _, odd in got] == [0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 0, 0]
+
+
+def test_kernel_of_each_layout(tmp_path):
+    """Which kernel a call takes, forward and backward, by length, type and layout (RowsMode 0:
+    aligned, 1: alike, 2: any), and a decode update by its state."""
+    code = r"""
+bf16, fp32 = 1, 2
+
+def both(L, dtype=bf16, B=4, D=512, W=4, seq=False, **kw):
+    fkw = {k: v[:2] if k in ("offsets", "pads") else v for k, v in kw.items()}
+    p = bwd_params(B, D, L, W, dtype, seq_stride=1 if seq else None, **kw)
+    assert bwd_typed(p) == 0
+    b = route(launches[0])
+    return [fwd(B, D, L, W, dtype, seq=seq, **fkw), b]
+
+result = {
+    "aligned": both(2048), "aligned with ids": both(2048, seq=True), "aligned fp32": both(2048, fp32),
+    "odd length": both(2041), "odd length, a vector more": both(1023), "odd length fp32": both(1023, fp32),
+    "no more segments than the aligned form": [both(L, D=48, B=2)[1] for L in (3071, 5119)],
+    "unlike": both(2048, offsets=(2, 4, 6)), "unlike rows": both(2041, pads=(1, 2, 3)),
+    "unlike fp32": both(2048, fp32, offsets=(4, 8, 12)),
+    "32 vectors": both(256), "33 vectors": both(264), "short, unlike": both(100, pads=(1, 2, 3)),
+    "channel-last": both(2048, layout="last"), "channel-last, odd": both(2048, D=513, layout="last"),
+    "one channel": both(2048, D=1, layout="last", dim_pad=7, dtype=bf16),
+    "strided": both(2048, layout="strided"), "fp32 width 9": both(2048, fp32, W=9),
+    "update": [update(8, 512, 4, bf16, S=3), update(8, 512, 4, bf16, S=4), update(8, 512, 9, bf16, S=8),
+               update(8, 512, 4, bf16, S=3, state="step"), update(8, 512, 4, bf16, S=6),
+               update(8, 512, 4, bf16, S=64, ring=True), update(256, 5120, 4, bf16, S=64, ring=True),
+               update(8, 512, 4, bf16, S=64, ring=True, tokens=8), update(8, 512, 4, bf16, S=63, ring=True)],
+}
+"""
+    got = _launch_spy.run(code, tmp_path)
+
+    def rows(f, b):
+        return [["fwd_rows_vec", f], ["bwd_rows_vec", b]]
+
+    short = [["fwd_rows_short", None], ["bwd_rows_short", None]]
+    last = [["fwd_cl", None], ["bwd_clw", None]]
+    generic = [["fwd_generic", None], ["bwd_generic", None]]
+    assert got == {
+        "aligned": rows(0, 0), "aligned with ids": rows(0, 0), "aligned fp32": rows(0, 0),
+        "odd length": rows(1, 1), "odd length, a vector more": rows(2, 2), "odd length fp32": rows(1, 1),
+        "no more segments than the aligned form": [["bwd_rows_vec", 1]] * 2,
+        "unlike": rows(2, 2), "unlike rows": rows(2, 2), "unlike fp32": rows(2, 2),
+        "32 vectors": short, "33 vectors": rows(0, 0), "short, unlike": short,
+        "channel-last": last, "channel-last, odd": last, "one channel": generic,
+        "strided": generic, "fp32 width 9": generic,
+        "update": ["update_dir", "update_dir", "update_lin", "update_step", "update_generic", "update_circ_vec",
+                   "update_ring", "update_ring", "update_circ"],
+    }

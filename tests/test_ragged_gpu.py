@@ -15,7 +15,7 @@ its neighbours), and are held to the oracle on the same inputs:
   outputs or gradients (the reference never reads past a row's ends).
 
 The host side of the choice (ragged rows keep the row kernels) is pinned on
-the CPU by the workspace sizes in test_abi.py.
+the CPU in test_launch_plan.py.
 """
 
 from __future__ import annotations
