@@ -338,8 +338,11 @@ __global__ void __launch_bounds__(256) fwd_cl(const FwdArgs a) {
     // order, so a row's outputs can then be computed as soon as that row has
     // arrived (us, rows first -> last: bf16 1 x 4096 x 8192 with seq_idx 30.0 ->
     // 26.8, 1536 x 2048 6.6 -> 5.6; fp32 4 x 2048 x 2000 27.0 -> 24.2). 16-bit
-    // types without seq_idx are quicker with the rows first below C3's size
-    // (4 x 2048 x 2000 15.8 against 16.3)
+    // types without seq_idx are quicker with the rows first in back-to-back
+    // launches of larger grids and even in single ones (first / last, bf16, W 4:
+    // 1 x 4096 x 8192 22.2 / 22.7, single 27.4 / 27.2; 4 x 2048 x 2000 13.0 / 13.7,
+    // 16.6 / 16.6; 1 x 4096 x 4096 12.3 / 12.9, 15.2 / 15.7), slower on small ones and
+    // at W 9 (1 x 1536 x 2048 6.0 / 5.6; W 9 1 x 4096 x 8192 26.5 / 25.9)
     constexpr bool PARAMS_FIRST = SEQ || sizeof(T) == 4;
     int32_t lid = 0;
     if constexpr (SEQ) {

@@ -17,15 +17,15 @@
 //                     entries and loads the channels' state span (S dwords)
 //                     directly, one load per span; no LDS; four wavefronts
 //                     (channel groups) per workgroup.
+//   update_lin     -- as update_dir for W > 5: one token, S == W-1, channel-contiguous x /
+//                     out and contiguous state rows: one wavefront per (batch
+//                     entry, 16 * EPV channels) moves the group's state and x
+//                     spans as consecutive 16-byte vectors and exchanges them
+//                     through LDS.
 //   update_step    -- linear mode, one token, state with unit channel stride (a
 //                     step's channels together, as causal_conv1d_varlen_states
 //                     returns it): a lane owns one dword of channels of every
 //                     step.
-//   update_lin     -- the same for W > 5: one token, S == W-1, channel-contiguous x /
-//                     out and contiguous state rows: one wavefront per (batch
-//                     entry, 16 * EPV channels) moves the group's state and x
-//                     spans as consecutive 16-byte vectors, one per lane at
-//                     W = 4, and exchanges them through LDS.
 //   update_circ_vec -- circular mode on contiguous state lines of whole
 //                     16-byte chunks: two adjacent lanes per (b, c) read the
 //                     two chunks that hold its window (one 32-byte access),
@@ -36,7 +36,7 @@
 //   update_circ    -- other circular cases with up to 8 new tokens; one thread
 //                     per (b, c) with all loads issued before any store.
 //   update_generic -- everything else; one thread per (b, c).
-// Both use the forward's tap loop (fma in k order, then SiLU), so a decode
+// All use the forward's tap loop (fma in k order, then SiLU), so a decode
 // loop reproduces the full forward bit for bit.
 #include "cc1d_internal.hpp"
 
