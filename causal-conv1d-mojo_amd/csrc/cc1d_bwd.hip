@@ -1,25 +1,34 @@
-// cc1d_bwd.hip -- backward entry points: dispatch on the dtype code to the
-// per-dtype launchers (cc1d_bwd_kernels.hpp, instantiated by
-// cc1d_bwd_{fp16,bf16,fp32}.hip), and the allocation-free typed backward
-// with its static device scratch.
+// cc1d_bwd.hip -- backward entry points: dispatch on the dtype code and the
+// width to their launchers (cc1d_bwd_kernels.hpp, instantiated by
+// cc1d_bwd_{fp16,bf16}{,_wide}.hip and cc1d_bwd_fp32.hip), and the
+// allocation-free typed backward with its static device scratch.
 #include <mutex>
 
 #include "cc1d_internal.hpp"
 
 namespace cc1d {
 
+// f of the dtype's tag and the width
+template <typename F> static int with_dtype_width(const cc1d_bwd_params& p, F&& f) {
+    return with_dtype(p.dtype, [&](auto tag) { return with_width(p.width, [&](auto wc) { return f(tag, wc); }); });
+}
+
 int launch_bwd(const cc1d_bwd_params& p, hipStream_t stream) {
-    return with_dtype(p.dtype, [&](auto tag) { return launch_bwd_dtype<decltype(tag)>(p, stream); });
+    return with_dtype_width(p, [&](auto tag, auto wc) {
+        return launch_bwd_width<decltype(tag), decltype(wc)::value>(p, stream);
+    });
 }
 
 int launch_bwd_typed(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream) {
-    return with_dtype(p.dtype, [&](auto tag) { return launch_bwd_typed_dtype<decltype(tag)>(p, g, stream); });
+    return with_dtype_width(p, [&](auto tag, auto wc) {
+        return launch_bwd_typed_width<decltype(tag), decltype(wc)::value>(p, g, stream);
+    });
 }
 
 int64_t bwd_workspace_floats(const cc1d_bwd_params& p) {
     int64_t n = -1;
-    with_dtype(p.dtype, [&](auto tag) {
-        n = bwd_workspace_floats_dtype<decltype(tag)>(p);
+    with_dtype_width(p, [&](auto tag, auto wc) {
+        n = bwd_workspace_floats_width<decltype(tag), decltype(wc)::value>(p);
         return (int)CC1D_OK;
     });
     return n;

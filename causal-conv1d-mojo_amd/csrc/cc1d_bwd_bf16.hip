@@ -1,11 +1,12 @@
-// cc1d_bwd_bf16.hip -- the backward kernels and launchers for bf16 storage
-// (one translation unit per dtype, so the three compile in parallel).
+// cc1d_bwd_bf16.hip -- the backward kernels and launchers for bf16 storage, widths 2 to 5
+// (one translation unit per dtype and half of the widths, so they compile in parallel).
 #include "cc1d_bwd_kernels.hpp"
 
 namespace cc1d {
 
-template int launch_bwd_dtype<bf16>(const cc1d_bwd_params&, hipStream_t);
-template int launch_bwd_typed_dtype<bf16>(const cc1d_bwd_params&, const cc1d_bwd_grads&, hipStream_t);
-template int64_t bwd_workspace_floats_dtype<bf16>(const cc1d_bwd_params&);
+CC1D_BWD_INSTANTIATE(bf16, 2)
+CC1D_BWD_INSTANTIATE(bf16, 3)
+CC1D_BWD_INSTANTIATE(bf16, 4)
+CC1D_BWD_INSTANTIATE(bf16, 5)
 
 }  // namespace cc1d

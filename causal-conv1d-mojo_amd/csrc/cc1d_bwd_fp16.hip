@@ -1,11 +1,12 @@
-// cc1d_bwd_fp16.hip -- the backward kernels and launchers for f16 storage
-// (one translation unit per dtype, so the three compile in parallel).
+// cc1d_bwd_fp16.hip -- the backward kernels and launchers for fp16 storage, widths 2 to 5
+// (one translation unit per dtype and half of the widths, so they compile in parallel).
 #include "cc1d_bwd_kernels.hpp"
 
 namespace cc1d {
 
-template int launch_bwd_dtype<f16>(const cc1d_bwd_params&, hipStream_t);
-template int launch_bwd_typed_dtype<f16>(const cc1d_bwd_params&, const cc1d_bwd_grads&, hipStream_t);
-template int64_t bwd_workspace_floats_dtype<f16>(const cc1d_bwd_params&);
+CC1D_BWD_INSTANTIATE(f16, 2)
+CC1D_BWD_INSTANTIATE(f16, 3)
+CC1D_BWD_INSTANTIATE(f16, 4)
+CC1D_BWD_INSTANTIATE(f16, 5)
 
 }  // namespace cc1d

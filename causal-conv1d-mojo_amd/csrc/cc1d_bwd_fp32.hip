@@ -1,11 +1,16 @@
 // cc1d_bwd_fp32.hip -- the backward kernels and launchers for float storage
-// (one translation unit per dtype, so the three compile in parallel).
+// (all widths: those above 5 have no row kernels).
 #include "cc1d_bwd_kernels.hpp"
 
 namespace cc1d {
 
-template int launch_bwd_dtype<float>(const cc1d_bwd_params&, hipStream_t);
-template int launch_bwd_typed_dtype<float>(const cc1d_bwd_params&, const cc1d_bwd_grads&, hipStream_t);
-template int64_t bwd_workspace_floats_dtype<float>(const cc1d_bwd_params&);
+CC1D_BWD_INSTANTIATE(float, 2)
+CC1D_BWD_INSTANTIATE(float, 3)
+CC1D_BWD_INSTANTIATE(float, 4)
+CC1D_BWD_INSTANTIATE(float, 5)
+CC1D_BWD_INSTANTIATE(float, 6)
+CC1D_BWD_INSTANTIATE(float, 7)
+CC1D_BWD_INSTANTIATE(float, 8)
+CC1D_BWD_INSTANTIATE(float, 9)
 
 }  // namespace cc1d

@@ -1,7 +1,7 @@
 // cc1d_bwd_kernels.hpp -- fused backward kernels for gfx950 and their launch
-// planning, templated on the storage type. Each cc1d_bwd_<dtype>.hip
-// instantiates them for one type (the types compile in parallel);
-// cc1d_bwd.hip dispatches on the dtype code.
+// planning, templated on the storage type and the width. Each
+// cc1d_bwd_<dtype>[_wide].hip instantiates them for one type and half of the
+// widths (they compile in parallel); cc1d_bwd.hip dispatches on both.
 //
 // Semantics (src/causal_conv1d_mojo/bwd_full_cpu/kernel.mojo:25-314):
 //   dpre[t] = dout[t] * silu'(pre[t]) (or dout[t] without SiLU); 0 for t
@@ -1867,68 +1867,61 @@ __global__ void __launch_bounds__(64) bwd_reduce_small(const RedArgs r) {
 
 }  // namespace
 
-// ---- per-dtype entry templates (instantiated by cc1d_bwd_<dtype>.hip) ----
+// ---- entry templates (instantiated by cc1d_bwd_<dtype>[_wide].hip) ----
 
-template <typename T>
-int launch_bwd_dtype(const cc1d_bwd_params& p, hipStream_t stream) {
-    return with_width(p.width, [&](auto wc) {
-        constexpr int W = decltype(wc)::value;
-        return with_flag(p.apply_silu != 0, [&](auto sc) {
-            const BwdPlan pl = plan_bwd<T, W>(p);
-            return launch_plan<T, W, decltype(sc)::value>(pl, p, stream);
-        });
+template <typename T, int W>
+int launch_bwd_width(const cc1d_bwd_params& p, hipStream_t stream) {
+    return with_flag(p.apply_silu != 0, [&](auto sc) {
+        const BwdPlan pl = plan_bwd<T, W>(p);
+        return launch_plan<T, W, decltype(sc)::value>(pl, p, stream);
     });
 }
 
-template <typename T>
-int64_t bwd_workspace_floats_dtype(const cc1d_bwd_params& p) {
-    int64_t n = -1;
-    with_width(p.width, [&](auto wc) {
-        constexpr int W = decltype(wc)::value;
-        n = reserved_floats<T, W>(p, plan_bwd<T, W>(p));
-        return (int)CC1D_OK;
-    });
-    return n;
+template <typename T, int W>
+int64_t bwd_workspace_floats_width(const cc1d_bwd_params& p) {
+    return reserved_floats<T, W>(p, plan_bwd<T, W>(p));
 }
 
-template <typename T>
-int launch_bwd_typed_dtype(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream) {
-    return with_width(p.width, [&](auto wc) {
-        constexpr int W = decltype(wc)::value;
-        return with_flag(p.apply_silu != 0, [&](auto sc) {
-            BwdPlan pl = plan_bwd<T, W>(p);
-            if (!plan_fits<T, W>(p, pl, g.workspace_floats)) return (int)CC1D_ERR_WORKSPACE;
-            if (g.workspace == nullptr) return (int)CC1D_ERR_NULL_POINTER;
-            pl.a.part = g.workspace;
-            const int st = launch_plan<T, W, decltype(sc)::value>(pl, p, stream);
-            if (st != CC1D_OK) return st;
-            RedArgs r;
-            r.part = g.workspace;
-            r.dweight = g.dweight;
-            r.dbias = g.dbias;
-            r.dweight_stride[0] = g.dweight_stride[0];
-            r.dweight_stride[1] = g.dweight_stride[1];
-            r.dbias_stride = g.dbias_stride;
-            r.batch = p.batch;
-            r.dim = p.dim;
-            r.nseg = pl.a.nseg;
-            r.groups = pl.a.groups;
-            r.nc = 64 * (pl.cpl > 0 ? pl.cpl : 1);
-            r.nout = pl.kind == kBwdCl ? pl.a.groups * r.nc * (W + 1) : p.dim * (W + 1);
-            const int64_t n = p.batch * pl.a.nseg;  // records per channel
-            const dim3 grid((unsigned)ceil_div(r.nout, 64));
-            if (n <= kRedSmall) {
-                const dim3 one(64);
-                if (pl.kind == kBwdRows) return launch(bwd_reduce_small<T, W, kBwdRows>, grid, one, stream, r);
-                if (pl.kind == kBwdCl) return launch(bwd_reduce_small<T, W, kBwdCl>, grid, one, stream, r);
-                return launch(bwd_reduce_small<T, W, kBwdGeneric>, grid, one, stream, r);
-            }
-            const dim3 threads(64 * (unsigned)(n < 16 ? n : 16));
-            if (pl.kind == kBwdRows) return launch(bwd_reduce<T, W, kBwdRows>, grid, threads, stream, r);
-            if (pl.kind == kBwdCl) return launch(bwd_reduce<T, W, kBwdCl>, grid, threads, stream, r);
-            return launch(bwd_reduce<T, W, kBwdGeneric>, grid, threads, stream, r);
-        });
+template <typename T, int W>
+int launch_bwd_typed_width(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream) {
+    return with_flag(p.apply_silu != 0, [&](auto sc) {
+        BwdPlan pl = plan_bwd<T, W>(p);
+        if (!plan_fits<T, W>(p, pl, g.workspace_floats)) return (int)CC1D_ERR_WORKSPACE;
+        if (g.workspace == nullptr) return (int)CC1D_ERR_NULL_POINTER;
+        pl.a.part = g.workspace;
+        const int st = launch_plan<T, W, decltype(sc)::value>(pl, p, stream);
+        if (st != CC1D_OK) return st;
+        RedArgs r;
+        r.part = g.workspace;
+        r.dweight = g.dweight;
+        r.dbias = g.dbias;
+        r.dweight_stride[0] = g.dweight_stride[0];
+        r.dweight_stride[1] = g.dweight_stride[1];
+        r.dbias_stride = g.dbias_stride;
+        r.batch = p.batch;
+        r.dim = p.dim;
+        r.nseg = pl.a.nseg;
+        r.groups = pl.a.groups;
+        r.nc = 64 * (pl.cpl > 0 ? pl.cpl : 1);
+        r.nout = pl.kind == kBwdCl ? pl.a.groups * r.nc * (W + 1) : p.dim * (W + 1);
+        const int64_t n = p.batch * pl.a.nseg;  // records per channel
+        const dim3 grid((unsigned)ceil_div(r.nout, 64));
+        if (n <= kRedSmall) {
+            const dim3 one(64);
+            if (pl.kind == kBwdRows) return launch(bwd_reduce_small<T, W, kBwdRows>, grid, one, stream, r);
+            if (pl.kind == kBwdCl) return launch(bwd_reduce_small<T, W, kBwdCl>, grid, one, stream, r);
+            return launch(bwd_reduce_small<T, W, kBwdGeneric>, grid, one, stream, r);
+        }
+        const dim3 threads(64 * (unsigned)(n < 16 ? n : 16));
+        if (pl.kind == kBwdRows) return launch(bwd_reduce<T, W, kBwdRows>, grid, threads, stream, r);
+        if (pl.kind == kBwdCl) return launch(bwd_reduce<T, W, kBwdCl>, grid, threads, stream, r);
+        return launch(bwd_reduce<T, W, kBwdGeneric>, grid, threads, stream, r);
     });
 }
+
+#define CC1D_BWD_INSTANTIATE(T, W)                                                                         \
+    template int launch_bwd_width<T, W>(const cc1d_bwd_params&, hipStream_t);                              \
+    template int launch_bwd_typed_width<T, W>(const cc1d_bwd_params&, const cc1d_bwd_grads&, hipStream_t); \
+    template int64_t bwd_workspace_floats_width<T, W>(const cc1d_bwd_params&);
 
 }  // namespace cc1d

@@ -22,11 +22,11 @@ int launch_bwd_typed(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStrea
 int launch_bwd_typed_noalloc(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream);
 constexpr int64_t kStaticWorkspaceFloats = CC1D_NOALLOC_WORKSPACE_FLOATS;
 int64_t bwd_workspace_floats(const cc1d_bwd_params& p);
-// per-dtype backward launchers (explicitly instantiated in cc1d_bwd_<dtype>.hip)
-template <typename T> int launch_bwd_dtype(const cc1d_bwd_params& p, hipStream_t stream);
-template <typename T>
-int launch_bwd_typed_dtype(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream);
-template <typename T> int64_t bwd_workspace_floats_dtype(const cc1d_bwd_params& p);
+// backward launchers of one dtype and width (explicitly instantiated in cc1d_bwd_<dtype>[_wide].hip)
+template <typename T, int W> int launch_bwd_width(const cc1d_bwd_params& p, hipStream_t stream);
+template <typename T, int W>
+int launch_bwd_typed_width(const cc1d_bwd_params& p, const cc1d_bwd_grads& g, hipStream_t stream);
+template <typename T, int W> int64_t bwd_workspace_floats_width(const cc1d_bwd_params& p);
 int launch_update(const cc1d_update_params& p, hipStream_t stream);
 int launch_varlen_states(const cc1d_varlen_params& p, hipStream_t stream);
 // element size of a varlen gather: elem_bytes, or the size of dtype when it is 0
